@@ -197,9 +197,11 @@ int svdq_w4a4_gemm(const void* qa, int operand, const void* sxp, const void* qwe
 
 /* Block tile of the W4A4 GEMM svdq_w4a4_gemm runs for a shape (no fused op): returns the tile's
  * column count, 256 (256 x 256 tiles, wave tile 128 x 64) or 128 (256 x 128 tiles), or 0 when the
- * shape takes another kernel (other operand formats and group sizes).  Both tilings give
+ * shape takes another kernel (other operand formats and group sizes, and shapes with so few of
+ * these tiles that 32 x 32 to 128 x 64 tiles run them in less time).  All tilings give
  * bit-identical outputs; the environment variable SVDQ_W4A4_TILES=256x128 or 256x256 overrides
- * the choice (the second only where M, N and K are multiples of 256).  No reference counterpart:
+ * the choice (the second only where M, N and K are multiples of 256), as do 32x32, 64x64 and
+ * 128x64.  No reference counterpart:
  * a host-side query for callers that report which kernel ran (bench.py, tests). */
 int svdq_w4a4_gemm_tile_cols(int M, int N, int K, int group, int operand);
 

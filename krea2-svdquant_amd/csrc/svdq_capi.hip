@@ -376,6 +376,7 @@ int svdq_w4a4_gemm(const void* qa, int operand, const void* sxp, const void* qwe
 
 int svdq_w4a4_gemm_tile_cols(int M, int N, int K, int group, int operand) {
   if (operand != SVDQ_OPERAND_E3M2 || !fast_group(group) || M <= 0 || N <= 0 || K <= 0 || K % group) return 0;
+  if (svdq::w4a4_small_tile(M, &N, 1, K, group) >= 0) return 0;
   return group == 64 && svdq::use_wide_tiles(M, N, K) ? 256 : 128;
 }
 
@@ -444,7 +445,10 @@ int svdq_w4a4_gemm_siblings(const svdq_w4a4_sibling* layers, int count, int oper
     tiles += ((M + 255) / 256) * ((l.N + 127) / 128);
   }
   gs.tile0[count] = tiles;
-  if (operand == SVDQ_OPERAND_E3M2 && fast_group(group) && K % 512 == 0)
+  int ns[SVDQ_MAX_SIBLINGS];
+  for (int i = 0; i < count; ++i) ns[i] = layers[i].N;
+  if (operand == SVDQ_OPERAND_E3M2 && fast_group(group) &&
+      (K % 512 == 0 || svdq::w4a4_small_tile(M, ns, count, K, group) >= 0))
     return launched(svdq::launch_w4a4_siblings(gs, group, out_f32 == 1, stream), "w4a4_gemm_siblings");
   // other formats, groups and K: one launch per layer, in order
   for (int i = 0; i < count; ++i)

@@ -298,38 +298,6 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, f32x16 (&acc)[2][2
 }
 
 // --------------------------------------------------------------------------- W4A4
-// Global -> LDS DMA (global_load_lds_dword / _dwordx4): lane L of the wave writes its 4 (16)
-// bytes from base + off at LDS address lds + 4 L (16 L); `lds` (wave-uniform) goes in M0, as
-// an operand, so the compiler owns that register.  Issued as inline asm so that the compiler
-// neither orders later LDS reads after it (it cannot tell the pipeline stages apart) nor
-// counts it in its own waits: the kernel waits explicitly.
-// Two hazards the compiler cannot see, because it does not look inside inline asm:
-//  * gfx9 requires 1 wait state between an SALU instruction that writes M0 and an LDS DMA that
-//    reads it.  The compiler writes M0 (`s_mov_b32 m0, sN`) right before the asm block, so every
-//    DMA starts with `s_nop 0`.
-//  * gfx9 requires 5 wait states between a VALU instruction that writes an SGPR and a VMEM
-//    instruction that reads it.  Under SGPR pressure the compiler restores a spilled base pointer
-//    with v_readlane right before a DMA, which then reads a stale address (builds where that
-//    happened faulted the GPU).  NOP = true starts the DMA with `s_nop 4` instead (5 wait states,
-//    about 2% of the e3m2 GEMM's time); the kernels whose build restores SGPRs before a DMA (the
-//    fused-epilogue variants) set it.
-// tests/test_dma_hazards.py walks every DMA of the built library back over all its predecessor
-// paths and fails if one can read a VALU-written SGPR within 5 wait states or an SALU-written M0
-// within 1.
-template <bool NOP = false>
-__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
-  if (NOP) asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
-  else asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
-}
-template <bool NOP = false>
-__device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
-  if (NOP) asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
-  else asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "{m0}"(lds) : "memory");
-}
-__device__ __forceinline__ uint32_t lds_offset(const void* p) {
-  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p);
-}
-
 // W4A4 GEMM (exact INT4-code products on the FP8 or INT8 MFMA).
 //
 // Block tile 256 x 128, 8 waves in a 4 x 2 grid, wave tile 64 x 64 = 2 x 2 sub-tiles of
@@ -2206,6 +2174,14 @@ hipError_t launch_w4a4(const GemmParams& p, int G, int mode, bool out_f32, hipSt
   SVDQ_W4A4(128, 1)
 #undef SVDQ_W4A4
   if (mode == 2) {
+    if (!p.epi) {
+      if (const int small = w4a4_small_tile(p.M, &p.N, 1, p.K, G); small >= 0) {
+        GemmSiblings one{};
+        one.count = 1;
+        one.layer[0] = p;
+        return launch_w4a4_small(one, G, small, out_f32, st);
+      }
+    }
     if (G == 64 && !p.epi && use_wide_tiles(p.M, p.N, p.K)) {
       const dim3 wgrid((unsigned)(((p.M + 255) / 256) * ((p.N + 255) / 256)));
       // ranks 64 .. 256 (LoRA adapters, larger SVD ranks): the low-rank term in LDS chunks
@@ -2253,6 +2229,10 @@ hipError_t launch_w4a4(const GemmParams& p, int G, int mode, bool out_f32, hipSt
 hipError_t launch_w4a4_siblings(const GemmSiblings& gs, int G, bool out_f32, hipStream_t st) {
   if (gs.count < 1 || gs.count > MAX_SIBLINGS) return hipErrorInvalidValue;
   const int K = gs.layer[0].K, M = gs.layer[0].M;
+  int ns[MAX_SIBLINGS];
+  for (int i = 0; i < gs.count; ++i) ns[i] = gs.layer[i].N;
+  if (const int small = w4a4_small_tile(M, ns, gs.count, K, G); small >= 0)
+    return launch_w4a4_small(gs, G, small, out_f32, st);
   int tiles = 0;
   for (int i = 0; i < gs.count; ++i) {
     const GemmParams& p = gs.layer[i];
