@@ -1,7 +1,7 @@
 """The gfx950 backend function: ``fn(x, state) -> y`` like reference
 ``kernels/triton/generic_int4.py:227-244`` (``svdquant_linear_triton_generic``).
 
-Two launches per layer forward:
+One operator (``svdq::linear``) per layer forward, two passes on the GPU:
 
 * W4A4  (``mode="w4a4"``):  ``svdq::act_quant`` (codes, scales, mid) -> ``svdq::w4a4_gemm``;
 * W4A16 (``mode="w4a16"``): ``svdq::act_quant`` (x_hat, mid)         -> ``svdq::w4a16_gemm``.
@@ -65,6 +65,12 @@ class PreparedLayer:
             codes = self.operands[operand] = ops.prepare_weight_operand(self.qweight, operand)
         return codes
 
+    def gemm_weights(self, operand: int) -> tuple[Tensor, Tensor]:
+        """Weight and scales as the GEMM of this operand format takes them (``OPERAND_NONE``: W4A16)."""
+        if operand == ops.OPERAND_NONE:
+            return self.qweight, self.weight_scales
+        return self.weight_operand(operand), self.weight_scale_pairs(operand)
+
     def weight_scale_pairs(self, operand: int) -> Tensor:
         pairs = self.scale_pairs.get(operand)
         if pairs is None:
@@ -95,6 +101,7 @@ def prepare_layer(state: SVDQuantLinearState, adapters: Sequence = (),
     dev = torch.device(device) if device is not None else state.qweight.device
     if dev.type != "cuda":
         raise RuntimeError("HIP gfx950 backend needs its state on a GPU device")
+    ops.load_native()   # here rather than in the first forward, which may be traced
     n, k = (int(v) for v in state.original_shape)
     qweight = state.qweight.to(dev).contiguous()
     if qweight.dtype != torch.uint8 or qweight.dim() != 2 or qweight.shape[0] != n:
@@ -158,12 +165,6 @@ def prepare_layer(state: SVDQuantLinearState, adapters: Sequence = (),
     )
 
 
-def _flatten(x: Tensor) -> tuple[Tensor, tuple[int, ...]]:
-    if x.ndim < 2:
-        raise ValueError(f"expected [..., K] activation, got shape {tuple(x.shape)}")
-    return x.reshape(-1, x.shape[-1]).contiguous(), tuple(x.shape[:-1])
-
-
 def _aligned(t: Tensor) -> Tensor:
     """``t`` itself when its storage starts on 16 bytes (the kernels' vector loads), else a copy."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
@@ -212,34 +213,24 @@ def forward_prepared(x: Tensor, prep: PreparedLayer, *, mode: str = "w4a4", out_
         raise TypeError(f"HIP gfx950 backend takes bfloat16 activations, got {x.dtype}")
     if x.device != prep.device:
         raise ValueError(f"activation on {x.device}, layer on {prep.device}")
-    x2, lead = _flatten(x)
-    k = x2.shape[1]
-    if k > prep.kp:
-        raise ValueError(f"activation K={k} exceeds packed weight K={prep.kp}")
-    if k != prep.kp:
-        x2 = _pad_cols(x2, prep.kp)
-    epi, aux2, vec2 = _epilogue_operands(epilogue, aux, vec, x2.shape[0], prep.n, x.device)
+    if x.ndim < 2:
+        raise ValueError(f"expected [..., K] activation, got shape {tuple(x.shape)}")
+    if x.shape[-1] > prep.kp:
+        raise ValueError(f"activation K={x.shape[-1]} exceeds packed weight K={prep.kp}")
+    epi, aux2, vec2 = 0, None, None
+    if epilogue != "none" or aux is not None or vec is not None:
+        epi, aux2, vec2 = _epilogue_operands(epilogue, aux, vec, math.prod(x.shape[:-1]), prep.n, x.device)
     if mode == "w4a4":
         if operand not in ops.OPERAND_NAMES:
             raise ValueError(f"operand must be 'e4m3', 'e3m2' or 'i8', got {operand!r}")
-        opc = ops.OPERAND_NAMES[operand]
-        generic = prep.group_size not in FAST_GROUPS
-        if generic:
-            # group sizes other than 64 / 128: the generic kernels, int8 operands quantized from x_hat
-            opc = ops.OPERAND_I8
-        qa, sx, _, _, mid = ops.act_quant(x2, prep.srs, prep.l2, prep.lora_down, prep.lora_mult,
-                                          prep.group_size, prep.rtp, opc, False, generic, exact_div, True)
-        y = ops.w4a4_gemm(qa, sx, prep.weight_operand(opc), prep.weight_scale_pairs(opc), mid, prep.l1cat,
-                          prep.bias, prep.group_size, opc, out_f32, epi, aux2, vec2)
+        # group sizes other than 64 / 128: the generic kernels, int8 operands quantized from x_hat
+        opc = ops.OPERAND_NAMES[operand] if prep.group_size in FAST_GROUPS else ops.OPERAND_I8
     elif mode == "w4a16":
-        _, _, _, xhat, mid = ops.act_quant(x2, prep.srs, prep.l2, prep.lora_down, prep.lora_mult,
-                                           prep.group_size, prep.rtp, ops.OPERAND_NONE, False, True,
-                                           exact_div)
-        y = ops.w4a16_gemm(xhat, prep.qweight, prep.weight_scales, mid, prep.l1cat, prep.bias,
-                           prep.group_size, out_f32, epi, aux2, vec2)
+        opc = ops.OPERAND_NONE
     else:
         raise ValueError(f"mode must be 'w4a4' or 'w4a16', got {mode!r}")
-    return y.reshape(*lead, prep.n)
+    return ops.linear(x, prep.srs, prep.l2, prep.lora_down, prep.lora_mult, prep.group_size, prep.rtp,
+                      *prep.gemm_weights(opc), prep.l1cat, prep.bias, opc, out_f32, exact_div, epi, aux2, vec2)
 
 
 def forward_prepared_siblings(x: Tensor, preps: Sequence[PreparedLayer], *, mode: str = "w4a4",
@@ -268,31 +259,16 @@ def forward_prepared_siblings(x: Tensor, preps: Sequence[PreparedLayer], *, mode
         raise ValueError(f"mode must be 'w4a4' or 'w4a16', got {mode!r}")
     if operand not in ops.OPERAND_NAMES:
         raise ValueError(f"operand must be 'e4m3', 'e3m2' or 'i8', got {operand!r}")
-    opc = ops.OPERAND_NAMES[operand]
-    x2, lead = _flatten(x)
-    if x2.shape[1] > p0.kp:
-        raise ValueError(f"activation K={x2.shape[1]} exceeds packed weight K={p0.kp}")
-    if x2.shape[1] != p0.kp:
-        x2 = _pad_cols(x2, p0.kp)
-    if mode == "w4a16":
-        acts = [ops.act_quant(x2, p.srs, p.l2, p.lora_down, p.lora_mult, p.group_size, p.rtp, ops.OPERAND_NONE,
-                              False, True, exact_div) for p in preps]
-        ys = ops.w4a16_gemm_siblings([a[3] for a in acts], [p.qweight for p in preps],
-                                     [p.weight_scales for p in preps], [a[4] for a in acts],
-                                     [p.l1cat for p in preps], [p.bias for p in preps], p0.group_size, out_f32)
-        return [y.reshape(*lead, p.n) for y, p in zip(ys, preps)]
-    if opc == ops.OPERAND_E3M2 and all(p.lora_down is None and p.rtp == p0.rtp for p in preps):
-        # one activation-pass launch for the layers (each its own smoothing) and one finalize
-        flat = ops.act_quant_siblings(x2, [p.srs for p in preps], [p.l2 for p in preps], p0.group_size, p0.rtp,
-                                      exact_div)
-        acts = [(flat[3 * i], flat[3 * i + 1], None, None, flat[3 * i + 2]) for i in range(len(preps))]
-    else:
-        acts = [ops.act_quant(x2, p.srs, p.l2, p.lora_down, p.lora_mult, p.group_size, p.rtp, opc, False, False,
-                              exact_div, True) for p in preps]
-    ys = ops.w4a4_gemm_siblings([a[0] for a in acts], [a[1] for a in acts], [p.weight_operand(opc) for p in preps],
-                                [p.weight_scale_pairs(opc) for p in preps], [a[4] for a in acts],
-                                [p.l1cat for p in preps], [p.bias for p in preps], p0.group_size, opc, out_f32)
-    return [y.reshape(*lead, p.n) for y, p in zip(ys, preps)]
+    if x.ndim < 2:
+        raise ValueError(f"expected [..., K] activation, got shape {tuple(x.shape)}")
+    if x.shape[-1] > p0.kp:
+        raise ValueError(f"activation K={x.shape[-1]} exceeds packed weight K={p0.kp}")
+    opc = ops.OPERAND_NAMES[operand] if mode == "w4a4" else ops.OPERAND_NONE
+    weights = [p.gemm_weights(opc) for p in preps]
+    return ops.linear_siblings(x, [p.srs for p in preps], [p.l2 for p in preps], [p.lora_down for p in preps],
+                               [p.lora_mult for p in preps], p0.group_size, [p.rtp for p in preps],
+                               [w for w, _ in weights], [s for _, s in weights], [p.l1cat for p in preps],
+                               [p.bias for p in preps], opc, out_f32, exact_div)
 
 
 # Prepared operands of the stateless entry, per state object: id(state) -> (key, PreparedLayer).  An

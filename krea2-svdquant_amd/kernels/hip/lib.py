@@ -16,6 +16,8 @@ import torch  # noqa: F401  (must precede the library load: HIP runtime binding)
 PKG_DIR = Path(__file__).resolve().parents[2]
 LIB_PATH = Path(os.environ.get("SVDQ_GFX950_LIB", PKG_DIR / "_lib" / "libsvdq_gfx950.so"))
 
+TORCH_LIB_PATH = PKG_DIR / "_lib" / "libsvdq_torch.so"
+
 SVDQ_ACT_PACKED = 1
 SVDQ_ACT_XHAT = 2
 SVDQ_ACT_EXACT_DIV = 4
@@ -96,7 +98,7 @@ SIGNATURES = {
                                       _P, _L, _P, _P]),
 }
 
-_lock = threading.Lock()
+lock = threading.RLock()
 _lib: ctypes.CDLL | None = None
 
 
@@ -113,7 +115,7 @@ def load() -> ctypes.CDLL:
     global _lib
     if _lib is not None:
         return _lib
-    with _lock:
+    with lock:
         if _lib is None:
             if not LIB_PATH.exists():
                 raise RuntimeError(
@@ -126,6 +128,15 @@ def load() -> ctypes.CDLL:
                 fn.argtypes = args
             _lib = lib
     return _lib
+
+
+def load_torch_ops() -> None:
+    """Load the native torch operators ``svdq::linear`` and ``svdq::linear_siblings``
+    (``csrc/svdq_torch.cpp``), which call this library; the caller holds ``lock``."""
+    load()
+    if not TORCH_LIB_PATH.exists():
+        raise RuntimeError(f"torch operators not found at {TORCH_LIB_PATH}; build them with __graft_entry__.build()")
+    torch.ops.load_library(str(TORCH_LIB_PATH))
 
 
 def call(name: str, *args) -> None:

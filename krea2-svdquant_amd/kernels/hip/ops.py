@@ -7,6 +7,7 @@ stream (no host synchronisation).  Fake (meta) implementations describe the outp
 from __future__ import annotations
 
 import ctypes
+import re
 from typing import Optional
 
 import torch
@@ -456,6 +457,59 @@ def w4a16_gemm_siblings(xhat: list[Tensor], qweight: list[Tensor], weight_scales
 def _(xhat, qweight, weight_scales, mid, l1cat, bias, group_size, out_f32):
     return [x.new_empty((x.shape[0], w.shape[0]), dtype=torch.float32 if out_f32 else torch.bfloat16)
             for x, w in zip(xhat, qweight)]
+
+
+# ---- whole linears: the native operators of csrc/svdq_torch.cpp ----------------------------------
+def _linear_fake(x, srs, l2, lora_down, lora_mult, group_size, rtp, weight, weight_scales, l1cat, bias, operand, out_f32, exact,
+      epi=0, aux=None, vec=None):
+    return x.new_empty((*x.shape[:-1], l1cat.shape[0]), dtype=torch.float32 if out_f32 else torch.bfloat16)
+
+
+def _linear_siblings_fake(x, srs, l2, lora_down, lora_mult, group_size, rtp, weight, weight_scales, l1cat, bias, operand, out_f32, exact):
+    return [x.new_empty((*x.shape[:-1], w.shape[0]), dtype=torch.float32 if out_f32 else torch.bfloat16)
+            for w in l1cat]
+
+
+_native_ops: dict = {}
+
+
+def load_native() -> dict:
+    """The native operators by name, loaded and given their shape functions on the first call."""
+    with lib.lock:
+        if not _native_ops:
+            lib.load_torch_ops()
+            torch.library.register_fake("svdq::linear", _linear_fake)
+            torch.library.register_fake("svdq::linear_siblings", _linear_siblings_fake)
+            _native_ops.update(linear=torch.ops.svdq.linear.default,
+                               linear_siblings=torch.ops.svdq.linear_siblings.default)
+    return _native_ops
+
+
+_STATUS_CODES = {name: code for code, name in lib.STATUS.items()}
+
+
+def _native(op: str, *args):
+    """Call a native operator; a C-ABI status comes back as ``SVDQError``, as from ``lib.call``."""
+    try:
+        return (_native_ops or load_native())[op](*args)
+    except RuntimeError as e:
+        m = re.match(r"(svdq_\w+) failed with (SVDQ_ERR_\w+): (.*)", str(e))
+        if m is None or m.group(2) not in _STATUS_CODES:
+            raise
+        raise lib.SVDQError(m.group(1), _STATUS_CODES[m.group(2)], m.group(3)) from e
+
+
+def linear(*args) -> Tensor:
+    """``svdq::linear``: one quantized linear, ``act_quant`` and ``w4a4_gemm`` (``operand`` one of the
+    W4A4 formats: ``weight`` its operand, ``weight_scales`` its scale pairs) or ``w4a16_gemm``
+    (``OPERAND_NONE``: the packed weight and its fp16 scales) on x [..., K], in one call."""
+    return _native("linear", *args)
+
+
+def linear_siblings(*args) -> list[Tensor]:
+    """``svdq::linear_siblings``: ``linear`` of sibling layers over one x, their activation passes and
+    GEMMs grouped as by ``act_quant_siblings``, ``w4a4_gemm_siblings`` and ``w4a16_gemm_siblings``."""
+    return _native("linear_siblings", *args)
 
 
 # ---- stand-in block normalizations -------------------------------------------------------------

@@ -117,12 +117,16 @@ class SVDQuantLinear(nn.Module):
 
     def _forward_base(self, x: torch.Tensor) -> torch.Tensor:
         """The quantized linear without LoRA adapters."""
-        return forward_prepared(x, self._prepare(x.device, with_adapters=False), mode=self._mode(x.device))
+        device = x.device
+        mode = self._mode(device)
+        return forward_prepared(x, self._prepared_for(device, with_adapters=False), mode=mode)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not self.lora_adapters:
             return self._forward_base(x)
-        return forward_prepared(x, self._prepare(x.device, with_adapters=True), mode=self._mode(x.device))
+        device = x.device
+        mode = self._mode(device)
+        return forward_prepared(x, self._prepared_for(device, with_adapters=True), mode=mode)
 
     def forward_epilogue(self, x: torch.Tensor, epilogue: str, aux: torch.Tensor,
                          vec: torch.Tensor | None = None) -> torch.Tensor:
@@ -152,8 +156,12 @@ class SVDQuantLinear(nn.Module):
 
     def _buffers_key(self, device: torch.device) -> tuple:
         # storage and version counter of every buffer: in-place edits bump the version
-        bufs = (self.qweight, self.smooth_scale, self.weight_scales, self.l1, self.l2, self.bias)
-        return (str(device),) + tuple((b.data_ptr(), b._version) if b is not None else None for b in bufs)
+        b = self._buffers
+        q, sm, ws, l1, l2, bias = (b["qweight"], b["smooth_scale"], b["weight_scales"], b["l1"], b["l2"],
+                                   b.get("bias"))
+        return (device, q.data_ptr(), q._version, sm.data_ptr(), sm._version, ws.data_ptr(), ws._version,
+                l1.data_ptr(), l1._version, l2.data_ptr(), l2._version,
+                None if bias is None else (bias.data_ptr(), bias._version))
 
     def _adapters_key(self) -> tuple:
         # each adapter's identity, multiplier (read on every forward, as the reference does) and
@@ -165,6 +173,9 @@ class SVDQuantLinear(nn.Module):
         """The kernels' operands of this layer, cached per (buffers, adapters).  The adapter entry
         shares the base entry's weight operands (prepare_layer's ``base``)."""
         self.resolved_backend(device)
+        return self._prepared_for(device, with_adapters)
+
+    def _prepared_for(self, device: torch.device, with_adapters: bool) -> PreparedLayer:
         base_key = self._buffers_key(device)
         hit = self._prepared.get(False)
         if hit is None or hit[0] != base_key:
