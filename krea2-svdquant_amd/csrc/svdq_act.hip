@@ -105,12 +105,23 @@ __device__ __forceinline__ void smooth64_exact(const u32x4 (&xr)[8], cfloat_ptr 
 // down-projected once per layer, in layer order, so that every layer's codes, scales and split
 // partials are bit-identical to its own pass (the same groups per wave, the same MFMA and
 // reduction order).
+// G = 128 (quantizing launches only: x_hat and the down projections do not depend on the group):
+// a group's two 64-column halves go to a pair of waves, which exchange their rows' maxima through
+// LDS, one barrier per pair of groups.  A wave then holds 64 columns as with G = 64 and two
+// workgroups share a CU; one wave with all 128 columns took 303-433 registers, one workgroup per
+// CU and a second round of workgroups: pass and finalize at M = 2381, K = 16384, rank 64 65.4 -> 37.1
+// us, M = 2381, K = 6144, rank 32 24.2 -> 17.6 us, M = 4096, K = 6144 with 64 + 64 ranks 69 -> 51 us.
+// The build is held to two workgroups per CU (256 registers; four rank tiles then spill, 51 against
+// 56 us without the limit).
 template <int G, int NT, int OPER, bool XHAT, bool QX, bool LX, int NL = 1>
 __device__ __forceinline__ void act_tile(const ActParams* lp) {
-  constexpr int HB = G / 64;             // 64-column blocks per group
-  constexpr bool QUANT = OPER != 0;
+  constexpr bool QUANT = OPER != 0, PAIR = G == 128;
+  static_assert(G == 64 || (G == 128 && QUANT), "groups of 128 matter to the quantizer only");
   static_assert(NL == 1 || (NT == 1 && !LX && !XHAT && !QX), "shared-x passes: one rank tile, codes only");
   __shared__ __attribute__((aligned(16))) float red[4 * 64 * 32];
+  __shared__ uint32_t pair_max[PAIR ? 2 : 1][4][64];   // |x_hat| maxima (bf16 bits) of each wave's rows
+  __shared__ uint32_t pair_bad[PAIR ? 2 : 1][4];
+  __shared__ float pair_exact[4][PAIR ? 64 : 1];
   const ActParams& p = lp[0];            // M, K, x and the split are the same for every layer
 
   const int tid = threadIdx.x;
@@ -124,6 +135,11 @@ __device__ __forceinline__ void act_tile(const ActParams* lp) {
   const int ngroups = K / G;
   const int gb = blockIdx.y * p.gps;
   const int ge = min(ngroups, gb + p.gps);
+  // the wave's groups: every 4th, or (pairs) every 2nd, every wave the same number of steps
+  constexpr int STEP = PAIR ? 2 : 4;
+  const int sub = PAIR ? wave & 1 : 0;   // the wave's half of its groups
+  const int g0 = gb + (PAIR ? wave >> 1 : wave);
+  const int gend = PAIR ? gb + (max(ge - gb, 0) + 1) / 2 * 2 : ge;
 
   f32x16 acc[NL][2][NT];
 #pragma unroll
@@ -138,38 +154,41 @@ __device__ __forceinline__ void act_tile(const ActParams* lp) {
   // stores and the low-rank MFMAs with no extra registers.  With LoRA the raw x feeds the LoRA
   // down projection, so each group is loaded when it starts.
   constexpr bool LORA = LX;
-  u32x4 xr[HB][8];
+  u32x4 xr[8];
   auto load_x = [&](int g) {
 #pragma unroll
-    for (int b = 0; b < HB; ++b)
-#pragma unroll
-      for (int c = 0; c < 8; ++c) xr[b][c] = ld16(p.x + rowc * p.ldx + g * G + 64 * b + 8 * c);
+    for (int c = 0; c < 8; ++c) xr[c] = ld16(p.x + rowc * p.ldx + g * G + 64 * sub + 8 * c);
   };
-  if (!LORA && gb + wave < ge) load_x(gb + wave);
-  for (int g = gb + wave; g < ge; g += 4) {
-    if (LORA) load_x(g);
+  int par = 0;
+  if (!LORA && g0 < ge) load_x(g0);
+  for (int g = g0; g < gend; g += STEP) {
+    const bool live = !PAIR || g < ge;   // (the last pair of an odd count of groups)
+    const int kb = g * G + 64 * sub;     // the wave's 64 columns
+    if (LORA && live) load_x(g);
 #pragma unroll
     for (int l = 0; l < NL; ++l) {
     const ActParams& p = lp[l];
     const int TR = (p.r + 31) >> 5;
     const cfloat_ptr sv = (cfloat_ptr)p.srs;
     const cfloat_ptr rv = (cfloat_ptr)(p.srs + K);
-    u32x4 xh[HB][8];
+    u32x4 xh[8];
+    float am = 0.0f;
 
     u16x2 amx = {0, 0}, xmx = {0, 0}, xmn = {0xFFFF, 0xFFFF};
-#pragma unroll
-    for (int b = 0; b < HB; ++b) smooth64_fast<XHAT>(xr[b], rv + g * G + 64 * b, xh[b], amx, xmx, xmn);
-    const uint32_t amb = amx[0] > amx[1] ? amx[0] : amx[1];
-    float am = bf16f((uint16_t)amb);
-    bool bad;
+    uint32_t amb = 0;
+    bool bad = false;
+    if (live) {
+    smooth64_fast<XHAT>(xr, rv + kb, xh, amx, xmx, xmn);
+    amb = amx[0] > amx[1] ? amx[0] : amx[1];
+    am = bf16f((uint16_t)amb);
     if (XHAT) {
       // x_hat needs every element exact: every nonzero quotient inside [2^-90, 2^100] (bounded by
       // the row's |x| range over the group's |s| range) and every s normal, so RN(1/s) is finite.
       // The s bit patterns are wave-uniform: scalar minimum / maximum.
       uint32_t smn = 0xFFFFFFFFu, smx = 0u;
 #pragma unroll
-      for (int j = 0; j < G; ++j) {
-        const uint32_t sb = __float_as_uint(sv[g * G + j]) & 0x7FFFFFFFu;
+      for (int j = 0; j < 64; ++j) {
+        const uint32_t sb = __float_as_uint(sv[kb + j]) & 0x7FFFFFFFu;
         smn = min(smn, sb);
         smx = max(smx, sb);
       }
@@ -181,83 +200,99 @@ __device__ __forceinline__ void act_tile(const ActParams* lp) {
       // Only codes and scales are written: they follow from the group absmax and, per element,
       // from the element's own quotient.  With the absmax inside [2^-90, 2^100] no quotient
       // leaves the range from above, and one below the normal range (< 2^-126, the only inexact
-      // case) is under 2^-33 of the scale, so its code is 0 either way.
+      // case) is under 2^-33 of the scale, so its code is 0 either way.  (A half of a group out of
+      // the range takes the division as well: the same results.)
       bad = amb != 0u && !(am >= 0x1p-90f && am <= 0x1p100f);
     }
-    if (p.exact || __any(bad)) {
-      am = 0.0f;
-#pragma unroll
-      for (int b = 0; b < HB; ++b) smooth64_exact(xr[b], sv + g * G + 64 * b, xh[b], am);
     }
-    if (l == NL - 1 && !LORA && g + 4 < ge) load_x(g + 4);
+    bool exact = p.exact || __any(bad);
+    if constexpr (PAIR) {
+      // the group's maximum over both halves; the division for the whole workgroup or for nobody, so
+      // that every wave meets the same barriers
+      pair_max[par][wave][lane] = amb;
+      if (lane == 0) pair_bad[par][wave] = exact;
+      __syncthreads();
+      am = bf16f((uint16_t)max(amb, pair_max[par][wave ^ 1][lane]));
+      exact = pair_bad[par][0] | pair_bad[par][1] | pair_bad[par][2] | pair_bad[par][3];
+      par ^= 1;
+    }
+    if (exact) {
+      am = 0.0f;
+      if (live) smooth64_exact(xr, sv + kb, xh, am);
+      if constexpr (PAIR) {
+        pair_exact[wave][lane] = am;
+        __syncthreads();
+        am = fmaxf(am, pair_exact[wave ^ 1][lane]);
+        __syncthreads();
+      }
+    }
+    if (l == NL - 1 && !LORA && g + STEP < ge) load_x(g + STEP);
+    if (!live) continue;
 
     if (QUANT) {
       const float sc = round_bf16(div_rcp(fmaxf(am, kBf16OneEMinus8), 7.0f, kRcp7));
       const float rsc = 1.0f / sc;
+      u32x4 op[4];
+      uint32_t nib[8];
+      f32x16 ex, ey;                      // OPER 3: the half's even-k and odd-k codes
 #pragma unroll
-      for (int b = 0; b < HB; ++b) {
-        u32x4 op[4];
-        uint32_t nib[8];
-        f32x16 ex, ey;                      // OPER 3: the half's even-k and odd-k codes
+      for (int c = 0; c < 8; ++c) {
+        float t[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          float t[8];
+        for (int e = 0; e < 4; ++e) {
+          // rint, then +0 turns -0 into +0 (canonical code bytes)
+          t[2 * e] = __builtin_rintf(div_rcp(bf16lo(xh[c][e]), sc, rsc)) + 0.0f;
+          t[2 * e + 1] = __builtin_rintf(div_rcp(bf16hi(xh[c][e]), sc, rsc)) + 0.0f;
+        }
+        if (OPER == 1) {
+          const uint32_t lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(
+              t[4], t[6], __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[2], 0, false), true);
+          const uint32_t hi = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(
+              t[5], t[7], __builtin_amdgcn_cvt_pk_fp8_f32(t[1], t[3], 0, false), true);
+          op[c >> 1][2 * (c & 1)] = lo;
+          op[c >> 1][2 * (c & 1) + 1] = hi;
+        }
+        if (OPER == 3) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            // rint, then +0 turns -0 into +0 (canonical code bytes)
-            t[2 * e] = __builtin_rintf(div_rcp(bf16lo(xh[b][c][e]), sc, rsc)) + 0.0f;
-            t[2 * e + 1] = __builtin_rintf(div_rcp(bf16hi(xh[b][c][e]), sc, rsc)) + 0.0f;
+            ex[4 * (c & 3) + e] = t[2 * e];
+            ey[4 * (c & 3) + e] = t[2 * e + 1];
           }
-          if (OPER == 1) {
-            const uint32_t lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(
-                t[4], t[6], __builtin_amdgcn_cvt_pk_fp8_f32(t[0], t[2], 0, false), true);
-            const uint32_t hi = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(
-                t[5], t[7], __builtin_amdgcn_cvt_pk_fp8_f32(t[1], t[3], 0, false), true);
-            op[c >> 1][2 * (c & 1)] = lo;
-            op[c >> 1][2 * (c & 1) + 1] = hi;
-          }
-          if (OPER == 3) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              ex[4 * (c & 3) + e] = t[2 * e];
-              ey[4 * (c & 3) + e] = t[2 * e + 1];
-            }
-            if ((c & 3) == 3 && rok) {
-              // k-step kt, half c / 4: 16 bytes to plane Q, 8 bytes to plane P
-              const u32x6 f = codes_to_e3m2(ex, ey);
-              const long mp = (p.M + 1) & ~1;      // plane rows, padded to even
-              const long plane = (long)((g * HB + b) * 2 + (c >> 2)) * mp + rowc;
-              *reinterpret_cast<u32x4*>(p.qa + plane * 16) = u32x4{f[0], f[1], f[2], f[3]};
-              *reinterpret_cast<u32x2*>(p.qa + mp * (K / 2) + plane * 8) = u32x2{f[4], f[5]};
-            }
-          }
-          if (OPER == 2 || (QX && p.qx)) {
-            uint32_t w = 0;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) w |= (uint32_t)((int)t[e] + 8) << (4 * e);
-            nib[c] = w;
-            if (OPER == 2) {
-              uint32_t lo, hi;
-              nib8_to_i8x16(w, lo, hi);
-              op[c >> 1][2 * (c & 1)] = lo;
-              op[c >> 1][2 * (c & 1) + 1] = hi;
-            }
+          if ((c & 3) == 3 && rok) {
+            // k-step kb / 64, half c / 4: 16 bytes to plane Q, 8 bytes to plane P
+            const u32x6 f = codes_to_e3m2(ex, ey);
+            const long mp = (p.M + 1) & ~1;      // plane rows, padded to even
+            const long plane = (long)(kb / 64 * 2 + (c >> 2)) * mp + rowc;
+            *reinterpret_cast<u32x4*>(p.qa + plane * 16) = u32x4{f[0], f[1], f[2], f[3]};
+            *reinterpret_cast<u32x2*>(p.qa + mp * (K / 2) + plane * 8) = u32x2{f[4], f[5]};
           }
         }
-        if (rok) {
-          if (OPER != 3) {
-            uint8_t* od = p.qa + rowc * K + g * G + 64 * b;
+        if (OPER == 2 || (QX && p.qx)) {
+          uint32_t w = 0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4*>(od + 16 * q) = op[q];
-          }
-          if (QX && p.qx) {
-            uint8_t* dst = p.qx + rowc * (K / 2) + (g * G + 64 * b) / 2;
-            *reinterpret_cast<u32x4*>(dst) = u32x4{nib[0], nib[1], nib[2], nib[3]};
-            *reinterpret_cast<u32x4*>(dst + 16) = u32x4{nib[4], nib[5], nib[6], nib[7]};
+          for (int e = 0; e < 8; ++e) w |= (uint32_t)((int)t[e] + 8) << (4 * e);
+          nib[c] = w;
+          if (OPER == 2) {
+            uint32_t lo, hi;
+            nib8_to_i8x16(w, lo, hi);
+            op[c >> 1][2 * (c & 1)] = lo;
+            op[c >> 1][2 * (c & 1) + 1] = hi;
           }
         }
       }
       if (rok) {
+        if (OPER != 3) {
+          uint8_t* od = p.qa + rowc * K + kb;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) *reinterpret_cast<u32x4*>(od + 16 * q) = op[q];
+        }
+        if (QX && p.qx) {
+          uint8_t* dst = p.qx + rowc * (K / 2) + kb / 2;
+          *reinterpret_cast<u32x4*>(dst) = u32x4{nib[0], nib[1], nib[2], nib[3]};
+          *reinterpret_cast<u32x4*>(dst + 16) = u32x4{nib[4], nib[5], nib[6], nib[7]};
+        }
+      }
+      if (rok && sub == 0) {
         const uint32_t sb = __float_as_uint(sc) >> 16;
         if (p.sx_pairs) reinterpret_cast<uint32_t*>(p.sx)[(long)g * p.M + rowc] = sb * 0x10001u;
         else p.sx[rowc * ngroups + g] = (uint16_t)sb;
@@ -265,50 +300,43 @@ __device__ __forceinline__ void act_tile(const ActParams* lp) {
     }
     if (XHAT && rok) {
 #pragma unroll
-      for (int b = 0; b < HB; ++b)
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-          *reinterpret_cast<u32x4*>(p.xhat + rowc * p.ldxh + g * G + 64 * b + 8 * c) = xh[b][c];
+      for (int c = 0; c < 8; ++c) *reinterpret_cast<u32x4*>(p.xhat + rowc * p.ldxh + kb + 8 * c) = xh[c];
     }
 
     // ---- low-rank down (x_hat @ L2^T) and LoRA down (x @ A^T) on MFMA, per 64 columns ----
+    // fa[i][c]: A operand of row tile i (rows 32i..32i+31) for the 16-column slice c
+    u32x4 fa[2][4], fx[2][4];
 #pragma unroll
-    for (int b = 0; b < HB; ++b) {
-      // fa[i][c]: A operand of row tile i (rows 32i..32i+31) for the 16-column slice c
-      u32x4 fa[2][4], fx[2][4];
+    for (int c = 0; c < 4; ++c) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          uint32_t v0 = xh[b][2 * c][d], v1 = xh[b][2 * c + 1][d];
-          permlane32_swap(v0, v1);
-          fa[0][c][d] = v0;
-          fa[1][c][d] = v1;
-          if (LX) {
-            uint32_t w0 = xr[b][2 * c][d], w1 = xr[b][2 * c + 1][d];
-            permlane32_swap(w0, w1);
-            fx[0][c][d] = w0;
-            fx[1][c][d] = w1;
-          }
+      for (int d = 0; d < 4; ++d) {
+        uint32_t v0 = xh[2 * c][d], v1 = xh[2 * c + 1][d];
+        permlane32_swap(v0, v1);
+        fa[0][c][d] = v0;
+        fa[1][c][d] = v1;
+        if (LX) {
+          uint32_t w0 = xr[2 * c][d], w1 = xr[2 * c + 1][d];
+          permlane32_swap(w0, w1);
+          fx[0][c][d] = w0;
+          fx[1][c][d] = w1;
         }
       }
-      const int kb = g * G + 64 * b;
+    }
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int T = p.t0 + t;   // global tile
-        const bool is_l2 = T < TR;
-        const int n = is_l2 ? 32 * T + lr : 32 * (T - TR) + lr;
-        const int nmax = is_l2 ? p.r : p.rl;
-        const uint16_t* bsrc = (is_l2 ? p.l2 : p.lora) + (long)min(n, nmax - 1) * K + kb + 8 * h;
-        const bool nok = n < nmax;
+    for (int t = 0; t < NT; ++t) {
+      const int T = p.t0 + t;   // global tile
+      const bool is_l2 = T < TR;
+      const int n = is_l2 ? 32 * T + lr : 32 * (T - TR) + lr;
+      const int nmax = is_l2 ? p.r : p.rl;
+      const uint16_t* bsrc = (is_l2 ? p.l2 : p.lora) + (long)min(n, nmax - 1) * K + kb + 8 * h;
+      const bool nok = n < nmax;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          u32x4 bf = ld16(bsrc + 16 * c);
-          if (!nok) bf = u32x4{};
+      for (int c = 0; c < 4; ++c) {
+        u32x4 bf = ld16(bsrc + 16 * c);
+        if (!nok) bf = u32x4{};
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
-            acc[l][i][t] = mfma_bf16_32x32x16(is_l2 ? fa[i][c] : fx[i][c], bf, acc[l][i][t]);
-        }
+        for (int i = 0; i < 2; ++i)
+          acc[l][i][t] = mfma_bf16_32x32x16(is_l2 ? fa[i][c] : fx[i][c], bf, acc[l][i][t]);
       }
     }
     }   // layers
@@ -357,7 +385,7 @@ __device__ __forceinline__ void act_tile(const ActParams* lp) {
 }
 
 template <int G, int NT, int OPER, bool XHAT, bool QX, bool LX>
-__global__ void __launch_bounds__(256) act_kernel(ActParams p) {
+__global__ void __launch_bounds__(256, G == 128 ? 2 : 1) act_kernel(ActParams p) {
   act_tile<G, NT, OPER, XHAT, QX, LX>(&p);
 }
 
@@ -377,49 +405,47 @@ __global__ void __launch_bounds__(256) act_shared_x_kernel(ActSiblings s) {
 
 // Final low-rank operand of the GEMM epilogue: the split partials summed in split order
 // (a fixed order, so the result is deterministic), then split into bf16 hi and lo planes
-// [M, 2, RTp] (the bf16 MFMA operands of mid @ l1cat^T).  One thread per 8 columns of a row.
+// [M, 2, RTp] (the bf16 MFMA operands of mid @ l1cat^T).  One thread per 4 columns of a row, eight
+// partials in flight: the launch is a few memory latencies long (M = 64, 24 splits: pass and finalize
+// 11.4 us with 8 columns per thread and four partials in flight, 8.8 us so).
+constexpr int kFinalizeThreads = 128;
 __device__ __forceinline__ void mid_finalize_rows(const float* __restrict__ part, int S, int M, int RTp,
                                                   uint16_t* __restrict__ midp) {
-  const int chunks = RTp / 8;
+  const int chunks = RTp / 4;
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= (long)M * chunks) return;
   const long m = idx / chunks;
   const int c = (int)(idx % chunks);
   const long plane = (long)M * RTp;
-  const float* src = part + m * RTp + 8 * c;
-  // the partials are loaded four splits at a time (past the last split the last one again, not
-  // added), then added in split order
-  f32x4 v0 = *reinterpret_cast<const f32x4*>(src), v1 = *reinterpret_cast<const f32x4*>(src + 4);
-  for (int s0 = 1; s0 < S; s0 += 4) {
-    f32x4 a0[4], a1[4];
+  const float* src = part + m * RTp + 4 * c;
+  // past the last split the last one again, not added
+  f32x4 v = *reinterpret_cast<const f32x4*>(src);
+  for (int s0 = 1; s0 < S; s0 += 8) {
+    f32x4 a[8];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const long o = (long)min(s0 + j, S - 1) * plane;
-      a0[j] = *reinterpret_cast<const f32x4*>(src + o);
-      a1[j] = *reinterpret_cast<const f32x4*>(src + o + 4);
-    }
+    for (int j = 0; j < 8; ++j) a[j] = *reinterpret_cast<const f32x4*>(src + (long)min(s0 + j, S - 1) * plane);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (s0 + j < S) {
-        v0 += a0[j];
-        v1 += a1[j];
-      }
+    for (int j = 0; j < 8; ++j)
+      if (s0 + j < S) v += a[j];
   }
-  const float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
-  u32x4 hi, lo;
-  split_hi_lo(v, hi, lo);
-  uint16_t* dst = midp + m * 2 * RTp + 8 * c;
-  *reinterpret_cast<u32x4*>(dst) = hi;
-  *reinterpret_cast<u32x4*>(dst + RTp) = lo;
+  u32x2 hi, lo;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
+    lo[i] = pack_bf16x2(v[2 * i] - bf16lo(hi[i]), v[2 * i + 1] - bf16hi(hi[i]));
+  }
+  uint16_t* dst = midp + m * 2 * RTp + 4 * c;
+  *reinterpret_cast<u32x2*>(dst) = hi;
+  *reinterpret_cast<u32x2*>(dst + RTp) = lo;
 }
 
-__global__ void __launch_bounds__(256) mid_finalize_kernel(const float* __restrict__ part, int S, int M, int RTp,
+__global__ void __launch_bounds__(kFinalizeThreads) mid_finalize_kernel(const float* __restrict__ part, int S, int M, int RTp,
                                                            uint16_t* __restrict__ midp) {
   mid_finalize_rows(part, S, M, RTp, midp);
 }
 
 // The finalize of sibling layers' passes in one launch (blockIdx.y = the layer).
-__global__ void __launch_bounds__(256) mid_finalize_siblings_kernel(ActSiblings s, int S) {
+__global__ void __launch_bounds__(kFinalizeThreads) mid_finalize_siblings_kernel(ActSiblings s, int S) {
   const ActParams& p = s.layer[blockIdx.y];
   mid_finalize_rows(p.mid, S, p.M, p.RTp, s.head[blockIdx.y]);
 }
@@ -497,7 +523,11 @@ hipError_t launch_act_nt(const ActParams& p, int nt, dim3 grid, hipStream_t st) 
   // L2); a down-projection-only launch may hold any mix
   switch (nt) {
     case 1: act_kernel<G, 1, OPER, XHAT, QX, MIDONLY><<<grid, 256, 0, st>>>(p); break;
-    case 2: act_kernel<G, 2, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p); break;
+    case 2:
+      // two rank tiles (ranks 33-64) without LoRA: x prefetched a group ahead as with one tile
+      if (!MIDONLY && p.rl == 0) act_kernel<G, 2, OPER, XHAT, QX, MIDONLY><<<grid, 256, 0, st>>>(p);
+      else act_kernel<G, 2, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p);
+      break;
     case 3: act_kernel<G, 3, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p); break;
     case 4: act_kernel<G, 4, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p); break;
     default: return hipErrorInvalidValue;
@@ -507,28 +537,26 @@ hipError_t launch_act_nt(const ActParams& p, int nt, dim3 grid, hipStream_t st) 
 
 template <int G>
 hipError_t launch_act_g(const ActParams& p, int nt, int oper, bool xhat, dim3 grid, hipStream_t st) {
-  if (p.t0 > 0) {   // down projections only
-    if (oper != 0 || xhat) return hipErrorInvalidValue;
-    return launch_act_nt<G, 0, false, false, true>(p, nt, grid, st);
+  if constexpr (G == 64) {   // independent of the group size
+    if (p.t0 > 0) return oper != 0 || xhat ? hipErrorInvalidValue : launch_act_nt<G, 0, false, false, true>(p, nt, grid, st);
+    if (oper == 0 && xhat) return launch_act_nt<G, 0, true, true>(p, nt, grid, st);
   }
   if (oper == 3 && !xhat && !p.qx) return launch_act_nt<G, 3, false, false>(p, nt, grid, st);
   if (oper == 3 && !xhat) return launch_act_nt<G, 3, false, true>(p, nt, grid, st);
   if (oper == 1 && !xhat) return launch_act_nt<G, 1, false, true>(p, nt, grid, st);
   if (oper == 1 && xhat) return launch_act_nt<G, 1, true, true>(p, nt, grid, st);
   if (oper == 2 && !xhat) return launch_act_nt<G, 2, false, true>(p, nt, grid, st);
-  if (oper == 0 && xhat) return launch_act_nt<G, 0, true, true>(p, nt, grid, st);
   return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-int act_splits(int M, int K, int G) {
+int act_splits(int M, int K) {
   // 512 workgroups fill the 256 CUs once (two 4-wave workgroups per CU): as many K splits as keep
   // row_tiles * splits within that, so no workgroups are left over for a second round
   const int row_tiles = (M + 63) / 64;
-  const int ngroups = K / G;
   int s = 512 / row_tiles;
-  const int smax = ngroups / 4 > 0 ? ngroups / 4 : 1;
+  const int smax = K / 256 > 0 ? K / 256 : 1;   // 64 columns for each of a workgroup's waves
   if (s > smax) s = smax;
   if (s < 1) s = 1;
   return s;
@@ -571,14 +599,16 @@ hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStrea
     else act_siblings_kernel<128><<<grid, 256, 0, st>>>(s);
   }
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  const long n = (long)s.layer[0].M * (s.layer[0].RTp / 8);
-  mid_finalize_siblings_kernel<<<dim3((unsigned)((n + 255) / 256), s.count), 256, 0, st>>>(s, splits);
+  const long n = (long)s.layer[0].M * (s.layer[0].RTp / 4);
+  const dim3 grid((unsigned)((n + kFinalizeThreads - 1) / kFinalizeThreads), s.count);
+  mid_finalize_siblings_kernel<<<grid, kFinalizeThreads, 0, st>>>(s, splits);
   return hipGetLastError();
 }
 
 hipError_t launch_mid_finalize(const float* part, int S, int M, int RTp, uint16_t* midp, hipStream_t st) {
-  const long n = (long)M * (RTp / 8);
-  mid_finalize_kernel<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(part, S, M, RTp, midp);
+  const long n = (long)M * (RTp / 4);
+  const unsigned blocks = (unsigned)((n + kFinalizeThreads - 1) / kFinalizeThreads);
+  mid_finalize_kernel<<<blocks, kFinalizeThreads, 0, st>>>(part, S, M, RTp, midp);
   return hipGetLastError();
 }
 

@@ -36,10 +36,10 @@ int launched(hipError_t e, const char* what) {
 
 bool fast_group(int group) { return group == 64 || group == 128; }
 
-// The group size the activation kernel runs with: the layer's own for 64 / 128; 64 for the generic
-// path (the kernel then writes x_hat and the down projections only, which do not depend on the
-// group, and the generic quantizer reads x_hat).
-int kernel_group(int group) { return fast_group(group) ? group : 64; }
+// The group size the activation kernel runs with: the layer's own where it quantizes (64 / 128);
+// 64 where it writes x_hat and the down projections only, which do not depend on the group (W4A16,
+// and the generic path, whose quantizer reads x_hat).
+int kernel_group(int group, bool quant) { return quant && fast_group(group) ? group : 64; }
 
 int check_group(int group, int K) {
   if (!svdq_group_supported(group))
@@ -73,7 +73,7 @@ int svdq_act_quant_workspace(int M, int K, int group, int RTp, int* splits, int6
   if (M <= 0) return fail(SVDQ_ERR_ARG, "act_quant_workspace: M=%d", M);
   if (int e = check_group(group, K)) return e;
   if (RTp <= 0 || RTp % 32) return fail(SVDQ_ERR_SHAPE, "RTp=%d must be a positive multiple of 32", RTp);
-  const int s = svdq::act_splits(M, K, kernel_group(group));
+  const int s = svdq::act_splits(M, K);
   if (splits) *splits = s;
   if (mid_floats) *mid_floats = (int64_t)(s + 1) * M * RTp;
   return ok();
@@ -147,7 +147,8 @@ int act_quant_run(const void* x, int64_t ldx, const float* srs, const void* l2, 
   p.xhat = static_cast<uint16_t*>(xhat);
   p.ldxh = ldxh;
   p.mid = part;
-  const int ngroups = K / kernel_group(group);   // the act kernel's groups
+  const int kgroup = kernel_group(group, quant);
+  const int ngroups = K / kgroup;   // the act kernel's groups
   p.gps = (ngroups + splits - 1) / splits;
   p.exact = (flags & SVDQ_ACT_EXACT_DIV) ? 1 : 0;
   p.sx_pairs = pairs ? 1 : 0;
@@ -165,7 +166,7 @@ int act_quant_run(const void* x, int64_t ldx, const float* srs, const void* l2, 
     q.qa = nullptr;
     q.sx = nullptr;
     q.qx = nullptr;
-    if (int e = launched(svdq::launch_act(q, kernel_group(group), nt < 4 ? nt : 4, 0, true, splits, stream),
+    if (int e = launched(svdq::launch_act(q, 64, nt < 4 ? nt : 4, 0, true, splits, stream),
                          "act_quant"))
       return e;
     if (i8) {
@@ -174,7 +175,7 @@ int act_quant_run(const void* x, int64_t ldx, const float* srs, const void* l2, 
                            "act_quant (any-group quantizer)"))
         return e;
     }
-  } else if (int e = launched(svdq::launch_act(p, group, nt < 4 ? nt : 4, e4m3 ? 1 : (i8 ? 2 : (e3m2 ? 3 : 0)),
+  } else if (int e = launched(svdq::launch_act(p, kgroup, nt < 4 ? nt : 4, e4m3 ? 1 : (i8 ? 2 : (e3m2 ? 3 : 0)),
                                                want_xhat, splits, stream),
                               "act_quant")) {
     return e;
@@ -182,11 +183,12 @@ int act_quant_run(const void* x, int64_t ldx, const float* srs, const void* l2, 
   for (int t0 = 4; t0 < nt; t0 += 4) {
     svdq::ActParams q = p;
     q.t0 = t0;
+    q.gps = p.gps * (kgroup / 64);   // the same columns in every split
     q.qa = nullptr;
     q.sx = nullptr;
     q.qx = nullptr;
     q.xhat = nullptr;
-    if (int e = launched(svdq::launch_act(q, kernel_group(group), nt - t0 < 4 ? nt - t0 : 4, 0, false, splits, stream),
+    if (int e = launched(svdq::launch_act(q, 64, nt - t0 < 4 ? nt - t0 : 4, 0, false, splits, stream),
                          "act_quant (down projections)"))
       return e;
   }
@@ -232,7 +234,7 @@ int svdq_act_quant(const void* x, int64_t ldx, const float* srs, const void* l2,
                    int RTp, unsigned flags, void* qa, void* sx, void* qx, void* xhat, int64_t ldxh,
                    float* mid, int splits, hipStream_t stream) {
   if (M > 0 && group > 0 && K > 0 && K % group == 0) {
-    const int expect = svdq::act_splits(M, K, kernel_group(group));
+    const int expect = svdq::act_splits(M, K);
     if (splits != expect) return fail(SVDQ_ERR_ARG, "act_quant: splits=%d, workspace says %d", splits, expect);
   }
   float* part = mid ? mid + (int64_t)(M > 0 ? M : 0) * (RTp > 0 ? RTp : 0) : nullptr;   // partials after the head
@@ -256,7 +258,7 @@ int svdq_act_quant_siblings(const void* x, int64_t ldx, const svdq_act_sibling* 
     }
     return SVDQ_OK;
   }
-  const int expect = svdq::act_splits(M, K, group);
+  const int expect = svdq::act_splits(M, K);
   if (M > 0 && splits != expect)
     return fail(SVDQ_ERR_ARG, "act_quant_siblings: splits=%d, workspace says %d", splits, expect);
   svdq::ActSiblings s{};
@@ -279,7 +281,7 @@ int svdq_act_quant_noalloc(const void* x, int64_t ldx, const float* srs, const v
   if (M <= 0) return fail(SVDQ_ERR_ARG, "act_quant_noalloc: M=%d", M);
   if (int e = check_group(group, K)) return e;
   if (RTp <= 0 || RTp % 32) return fail(SVDQ_ERR_SHAPE, "act_quant_noalloc: RTp=%d must be a positive multiple of 32", RTp);
-  const int splits = svdq::act_splits(M, K, kernel_group(group));
+  const int splits = svdq::act_splits(M, K);
   const int64_t need = (int64_t)splits * M * RTp;
   if (need > kScratchFloats)
     return fail(SVDQ_ERR_SHAPE,

@@ -144,16 +144,6 @@ __device__ __forceinline__ void permlane32_swap(uint32_t& a, uint32_t& b) {
   b = r[1];
 }
 
-// Split 8 floats into bf16 hi + bf16 lo parts (x ~= hi + lo to ~2^-17 relative).
-__device__ __forceinline__ void split_hi_lo(const float* v, u32x4& hi, u32x4& lo) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t h = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    hi[i] = h;
-    lo[i] = pack_bf16x2(v[2 * i] - bf16lo(h), v[2 * i + 1] - bf16hi(h));
-  }
-}
-
 // VGPR banks of the rescale FMA acc += P * S.  The FMA reads three VGPRs; the register file
 // has four banks (register index mod 4) and three operands in one bank issue at about half
 // rate (measured: 1.85x the time of three distinct banks).  The allocator starts the MFMA result

@@ -72,10 +72,10 @@ struct ActSiblings {
 };
 hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStream_t st);
 
-int act_splits(int M, int K, int G);
+int act_splits(int M, int K);
 // oper: 0 = no codes (x_hat only), 1 = e4m3 operand codes, 2 = int8 16*q operand codes, 3 = e3m2;
 // nt: column tiles of the down projections from p.t0 (at most 4); with p.t0 > 0 the launch computes
-// down projections only (oper 0, no x_hat)
+// down projections only (oper 0, no x_hat); launches without codes take G = 64
 hipError_t launch_act(const ActParams& p, int G, int nt, int oper, bool xhat, int splits, hipStream_t st);
 // Sums the S split partials `part` [S, M, RTp] in split order and writes the GEMM epilogue's
 // operand midp [M, 2, RTp] (bf16 hi plane, then bf16 lo plane, hi + lo within 2^-18 of the f32 sum, relative).

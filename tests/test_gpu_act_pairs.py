@@ -1,0 +1,38 @@
+"""GPU tests of the activation pass with groups of 128, whose halves go to a pair of waves: codes and
+scales bit-exact against the oracle quantizer with odd and even group counts per split, values that
+leave the smoothing's fast range in one half of a group only, and every rank tile count."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import sim, synth
+from .gpu_util import bf16_tensor, e3m2_codes_of, operand_bytes, sx_pairs_ok, to_device_state
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("m,k,rank,extreme", [(1, 128, 32, False), (3, 384, 64, False), (64, 640, 32, True),
+                                              (65, 1280, 64, True), (130, 6144, 96, False), (700, 1920, 128, True)])
+def test_codes_scales_and_down_projection(dev, m, k, rank, extreme):
+    from krea2_svdquant_amd.kernels.hip import backend, ops
+    x = synth.make_activation(m, k, seed=m + k)
+    if extreme:   # one half of some groups below 2^-90, above 2^100, or zero
+        x[:, 64:128] *= np.float32(2.0 ** -100)
+        x[0, 256:320] = np.float32(2.0 ** 105)
+        x[m // 2, 128:192] = 0.0
+    st = synth.make_layer(64, k, np.clip(x, -100, 100), rank=rank, group_size=128, seed=3)
+    prep = backend.prepare_layer(to_device_state(st, dev), (), dev)
+    xd = bf16_tensor(x, dev)
+    x_hat, _, sx_ref, codes = sim.quantize_activations(x, st)
+    for fmt, op in (("e3m2", ops.OPERAND_E3M2), ("i8", ops.OPERAND_I8)):
+        qa, sxp, _, _, mid = ops.act_quant(xd, prep.srs, prep.l2, None, None, 128, prep.rtp, op, False, False, False,
+                                           True)
+        got = qa.cpu().numpy()
+        assert np.array_equal(e3m2_codes_of(got, m, k) if fmt == "e3m2" else got,
+                              codes if fmt == "e3m2" else operand_bytes(codes, fmt))
+        assert sx_pairs_ok(sxp, sx_ref)
+        # f32 sums of K products in another order: K 2^-24 of the sum of magnitudes
+        want = np.asarray(x_hat, np.float64) @ np.asarray(st.l2, np.float64).T
+        bound = np.abs(np.asarray(x_hat, np.float64)) @ np.abs(np.asarray(st.l2, np.float64)).T * (k * 2.0 ** -24 + 2.0 ** -16)
+        err = np.abs(ops.mid_values(mid).cpu().numpy()[:, :rank] - want)
+        assert np.all(err <= bound + 1e-30)
