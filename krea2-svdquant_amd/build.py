@@ -19,7 +19,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libsvdq_gfx950.so"
 TORCH_LIB_PATH = LIB_DIR / "libsvdq_torch.so"
-SOURCES = ["svdq_act.hip", "svdq_gemm.hip", "svdq_gemm_small.hip", "svdq_block.hip", "svdq_attn.hip", "svdq_capi.hip"]
+SOURCES = ["svdq_act.hip", "svdq_gemm.hip", "svdq_gemm_small.hip", "svdq_w4a16_direct.hip", "svdq_block.hip", "svdq_attn.hip", "svdq_capi.hip"]
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [

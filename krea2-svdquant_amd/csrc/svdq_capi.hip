@@ -601,7 +601,7 @@ int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M,
   svdq::GemmSiblings gs{};
   gs.count = count;
   int tiles = 0;
-  bool fits = fast_group(group);
+  long own = 0;   // cost of a launch per layer
   for (int i = 0; i < count; ++i) {
     const svdq_w4a16_sibling& l = layers[i];
     if (int e = gemm_common_checks("w4a16_gemm_siblings", l.qw, l.sw, l.mid, l.l1cat, l.RTp, M, l.N, K, group, l.y,
@@ -615,13 +615,18 @@ int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M,
     p = gemm_params(l.qw, l.sw, l.mid, l.l1cat, l.RTp, l.bias, M, l.N, K, l.y, l.ldy);
     p.xhat = static_cast<const uint16_t*>(l.xhat);
     p.ldxh = l.ldxh;
-    fits = fits && svdq::w4a16_ws_fits(p);
+    svdq::GemmSiblings one{};
+    one.count = 1;
+    one.layer[0] = p;
+    own += svdq::w4a16_route(one).cost;
     gs.tile0[i] = tiles;
     tiles += ((M + 191) / 192) * ((l.N + 255) / 256);
   }
   gs.tile0[count] = tiles;
-  if (fits && svdq::w4a16_siblings_pay(gs))
-    return launched(svdq::launch_w4a16_siblings(gs, group, out_f32 == 1, stream), "w4a16_gemm_siblings");
+  if (const svdq::W4A16Route r = svdq::w4a16_route(gs); fast_group(group) && r.tile != svdq::W4A16_WIDE && r.cost <= own)
+    return launched(r.tile == svdq::W4A16_WS ? svdq::launch_w4a16_siblings(gs, group, out_f32 == 1, stream)
+                                             : svdq::launch_w4a16_direct(gs, group, r.tile, out_f32 == 1, stream),
+                    "w4a16_gemm_siblings");
   // otherwise one launch per layer, in order, each with its own tile choice
   for (int i = 0; i < count; ++i)
     if (int e = launched(svdq::launch_w4a16(gs.layer[i], group, out_f32 == 1, stream), "w4a16_gemm_siblings"))

@@ -2324,29 +2324,14 @@ hipError_t launch_weight_operand(const uint8_t* qw, uint8_t* qwe, int N, int K, 
 }
 
 // The specialized-wave kernel takes a layer without a fused op whose x_hat rows are 16-byte
-// aligned and whose DMA offsets fit 32 bits, unless SVDQ_W4A16_KERNEL=wide.
+// aligned and whose DMA offsets fit 32 bits (a row's byte offset from the x_hat base and from the mid
+// planes'; larger operands go to kernels that address rows or tiles in 64 bits), unless
+// SVDQ_W4A16_KERNEL=wide.
 bool w4a16_ws_fits(const GemmParams& p) {
   const char* ke = getenv("SVDQ_W4A16_KERNEL");
   const bool xa = (reinterpret_cast<uintptr_t>(p.xhat) & 15) == 0 && p.ldxh % 8 == 0;
   const bool off32 = ((long)p.M - 1) * p.ldxh * 2 + 128 <= 0xFFFFFFFFL && (long)p.M * 4 * p.RTp <= 0xFFFFFFFFL;
   return !p.epi && xa && off32 && !(ke && !strcmp(ke, "wide"));
-}
-
-// Sibling layers on one launch of 192 x 256 tiles pay when their rounds over the 256 CUs cost no
-// more than the layers' own launches.  Cost of a round = its tile height in rows (time per tile at
-// a given K grows with the rows: 142 / 187 us for 192 / 256 rows at K = 6144); the 128 x 128
-// kernel's rounds (one 4-wave workgroup per CU) count 110, its measured 82 us against 142.
-bool w4a16_siblings_pay(const GemmSiblings& gs) {
-  long own = 0, t192 = 0;
-  for (int i = 0; i < gs.count; ++i) {
-    const GemmParams& p = gs.layer[i];
-    const long nb256 = (p.N + 255) / 256, tw = (long)((p.M + 255) / 256) * nb256;
-    const long t = (long)((p.M + 191) / 192) * nb256;
-    t192 += t;
-    if (tw >= 128) own += std::min((t + 255) / 256 * 192, (tw + 255) / 256 * 256);
-    else own += ((long)((p.M + 127) / 128) * ((p.N + 127) / 128) + 255) / 256 * 110;
-  }
-  return (t192 + 255) / 256 * 192 <= own;
 }
 
 hipError_t launch_w4a16_siblings(const GemmSiblings& gs, int G, bool out_f32, hipStream_t st) {
@@ -2382,16 +2367,41 @@ hipError_t launch_w4a16(const GemmParams& p, int G, bool out_f32, hipStream_t st
     else w4a16_kernel<0, 2, false><<<grid, 256, 0, st>>>(q);
     return hipGetLastError();
   }
-  // 256 x 256 tiles (one wave per SIMD) when they cover the chip at least half, else 128 x 128
-  // tiles (two workgroups of 4 waves per CU)
+  const char* ke = getenv("SVDQ_W4A16_KERNEL");
   const long nbn = (p.N + 255) / 256;
-  const long tiles_wide = (long)((p.M + 255) / 256) * nbn;
-  if (tiles_wide >= 128) {
-    // tile height 256 or 192: the one with the least work per CU, rounds of tiles x tile rows (a
-    // round = one tile on each of the 256 CUs); e.g. M = 2304, N = 16384: 576 tiles of 256 rows
-    // need 3 rounds (the last a quarter full), 768 tiles of 192 rows 3 full rounds
-    const long tiles192 = (long)((p.M + 191) / 192) * nbn;
-    const bool t192 = ((tiles192 + 255) / 256) * 192 < ((tiles_wide + 255) / 256) * 256;
+  const long tiles_wide = (long)((p.M + 255) / 256) * nbn, tiles192 = (long)((p.M + 191) / 192) * nbn;
+  int route = W4A16_WIDE;
+  if (p.epi || (ke && !strcmp(ke, "wide") && tiles_wide >= 128)) {
+    // Register-staged tiles: with a fused op, and by the environment (tests compare the others with them).
+    if (tiles_wide < 128) {
+      // 128 x 128 (two workgroups of 4 waves per CU) when 256 x 256 tiles leave half the chip idle
+      const dim3 grid(((p.M + 127) / 128) * ((p.N + 127) / 128));
+      if (G == 64) w4a16_kernel<64, 2, false, true><<<grid, 256, 0, st>>>(p);
+      else w4a16_kernel<128, 2, false, true><<<grid, 256, 0, st>>>(p);
+      return hipGetLastError();
+    }
+  } else {
+    GemmSiblings one{};
+    one.count = 1;
+    one.layer[0] = p;
+    route = w4a16_route(one).tile;
+    if (route >= 0) return launch_w4a16_direct(one, G, route, out_f32, st);
+    if (route == W4A16_WS) {
+      const dim3 grid((unsigned)tiles192);
+      if (G == 64) {
+        if (out_f32) w4a16_ws_kernel<64, true><<<grid, 512, 0, st>>>(p);
+        else w4a16_ws_kernel<64, false><<<grid, 512, 0, st>>>(p);
+      } else {
+        if (out_f32) w4a16_ws_kernel<128, true><<<grid, 512, 0, st>>>(p);
+        else w4a16_ws_kernel<128, false><<<grid, 512, 0, st>>>(p);
+      }
+      return hipGetLastError();
+    }
+  }
+  // tile height 256 or 192: the one with the least work per CU, rounds of tiles x tile rows (a
+  // round = one tile on each of the 256 CUs); e.g. M = 2304, N = 16384: 576 tiles of 256 rows
+  // need 3 rounds (the last a quarter full), 768 tiles of 192 rows 3 full rounds
+  const bool t192 = ((tiles192 + 255) / 256) * 192 < ((tiles_wide + 255) / 256) * 256;
 #define SVDQ_W4A16W(GG, TT)                                                                 \
   if (G == GG) {                                                                            \
     const dim3 grid((unsigned)(TT == 192 ? tiles192 : tiles_wide));                         \
@@ -2400,44 +2410,14 @@ hipError_t launch_w4a16(const GemmParams& p, int G, bool out_f32, hipStream_t st
     else w4a16_wide_kernel<GG, false, false, TT><<<grid, 256, 0, st>>>(p);                  \
     return hipGetLastError();                                                               \
   }
-    // the 192-row tiles on specialized waves (w4a16_ws_kernel; its x_hat DMA moves 16-byte chunks:
-    // rows 16-byte aligned) unless SVDQ_W4A16_KERNEL=wide.  Its DMA addresses a row by a 32-bit
-    // byte offset from the x_hat base (row * ldxh * 2) and from the mid planes' (row * 4 * RTp):
-    // larger operands take the register-staged kernel, which addresses rows in 64 bits.
-    if (t192 && w4a16_ws_fits(p)) {
-      const dim3 grid((unsigned)tiles192);
-      if (G == 64) {
-        if (out_f32) w4a16_ws_kernel<64, true><<<grid, 512, 0, st>>>(p);
-        else w4a16_ws_kernel<64, false><<<grid, 512, 0, st>>>(p);
-        return hipGetLastError();
-      }
-      if (G == 128) {
-        if (out_f32) w4a16_ws_kernel<128, true><<<grid, 512, 0, st>>>(p);
-        else w4a16_ws_kernel<128, false><<<grid, 512, 0, st>>>(p);
-        return hipGetLastError();
-      }
-    }
-    if (t192) {
-      SVDQ_W4A16W(64, 192)
-      SVDQ_W4A16W(128, 192)
-    } else {
-      SVDQ_W4A16W(64, 256)
-      SVDQ_W4A16W(128, 256)
-    }
+  if (t192) {
+    SVDQ_W4A16W(64, 192)
+    SVDQ_W4A16W(128, 192)
+  } else {
+    SVDQ_W4A16W(64, 256)
+    SVDQ_W4A16W(128, 256)
+  }
 #undef SVDQ_W4A16W
-    return hipErrorInvalidValue;
-  }
-  const dim3 grid(((p.M + 127) / 128) * ((p.N + 127) / 128));
-#define SVDQ_W4A16(GG)                                                                     \
-  if (G == GG) {                                                                          \
-    if (out_f32) w4a16_kernel<GG, 2, true><<<grid, 256, 0, st>>>(p);                       \
-    else if (p.epi) w4a16_kernel<GG, 2, false, true><<<grid, 256, 0, st>>>(p);             \
-    else w4a16_kernel<GG, 2, false><<<grid, 256, 0, st>>>(p);                              \
-    return hipGetLastError();                                                             \
-  }
-  SVDQ_W4A16(64)
-  SVDQ_W4A16(128)
-#undef SVDQ_W4A16
   return hipErrorInvalidValue;
 }
 

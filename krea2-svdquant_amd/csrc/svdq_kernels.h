@@ -105,11 +105,19 @@ hipError_t launch_weight_scale_pairs(const uint16_t* sw, uint32_t* out, int n, i
 // bytes per row)
 hipError_t launch_weight_operand(const uint8_t* qw, uint8_t* qwe, int N, int K, int mode, hipStream_t st);
 hipError_t launch_w4a16(const GemmParams& p, int G, bool out_f32, hipStream_t st);
-// W4A16 sibling layers (same M, K and group; tile0 counting 192 x 256 tiles) in one launch of the
+// Which kernel runs W4A16 layers over the same rows (no fused op, group 64 or 128) in one launch, by the
+// cost of its rounds of tiles, and that cost: a tile of svdq_w4a16_direct.hip (>= 0), the specialized
+// waves, or (a single layer) the 256-row register-staged tiles.
+constexpr int W4A16_WS = -1, W4A16_WIDE = -2;
+struct W4A16Route {
+  int tile;
+  long cost;
+};
+W4A16Route w4a16_route(const GemmSiblings& gs);
+hipError_t launch_w4a16_direct(const GemmSiblings& gs, int G, int tile, bool out_f32, hipStream_t st);
+// Sibling layers (tile0 in 192 x 256 tiles, filled in by the caller) in one launch of the
 // specialized-wave kernel; hipErrorInvalidValue when a layer cannot take it (w4a16_ws_fits).
-// w4a16_siblings_pay: whether that launch beats the layers' own launches (their tile rounds).
 bool w4a16_ws_fits(const GemmParams& p);
-bool w4a16_siblings_pay(const GemmSiblings& gs);
 hipError_t launch_w4a16_siblings(const GemmSiblings& gs, int G, bool out_f32, hipStream_t st);
 // W4A4 GEMM for any group size G (multiple of 16 dividing K): int8 operands (SVDQ_OPERAND_I8 layout)
 hipError_t launch_w4a4_any_group(const GemmParams& p, int G, bool out_f32, hipStream_t st);
