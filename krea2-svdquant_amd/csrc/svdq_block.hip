@@ -40,6 +40,12 @@ __device__ __forceinline__ u32x4 addcmul8(u32x4 x, u32x4 g, u32x4 v) {
 // pass 2 writes the normalized, weighted and shifted chunks (chunks beyond NR re-read from L2).
 // RES: the row is first formed as the gated residual x + g * v (g a vector [H], v the layer output
 // [T, ldv]) and written to xo, and that row is normalized (chunks beyond NR re-read from xo).
+// HBM-bound, two reads and two writes per value (RES).  NR is the row's own chunk count, so a row of 6144
+// keeps three chunks and not four, and the stores are non-temporal: lines that are written once leave the
+// L2s to the rows still being read.  RES, T = 4352, H = 6144, launches back to back over four sets of buffers:
+// 44.2 us (4.84 TB/s; a copy of the same streams 43.4) -> 41.7 with NR = 3 -> 39.7 (5.40 TB/s); through the
+// torch operator 44.4 -> 42.0; T = 16384: 149.6 -> 139.2; T = 128: 3.93 -> 3.70.  No gain:
+// non-temporal loads as well (1101 rows 10.5 -> 12.1), 512 workgroups of several rows each (T = 16384: 144).
 template <int NR, bool RES = false>
 __global__ void __launch_bounds__(256) rms_norm_modulate_kernel(const uint16_t* __restrict__ x, long ldx,
                                                                 const uint16_t* __restrict__ w,
@@ -52,11 +58,13 @@ __global__ void __launch_bounds__(256) rms_norm_modulate_kernel(const uint16_t* 
   const int tid = threadIdx.x, nc = H / 8;
   const uint16_t* xr = x + (long)blockIdx.x * ldx;
   uint16_t* xor_ = RES ? xo + (long)blockIdx.x * ldxo : nullptr;
-  auto row_chunk = [&](int c) {   // the chunk to normalize (RES: formed and stored first)
+  // the chunk to normalize (RES: formed and stored first; again: it will be re-read)
+  auto row_chunk = [&](int c, bool again) {
     u32x4 r = ld16(xr + 8 * c);
     if (RES) {
       r = addcmul8(r, ld16(g + 8 * c), ld16(v + (long)blockIdx.x * ldv + 8 * c));
-      *reinterpret_cast<u32x4*>(xor_ + 8 * c) = r;
+      if (again) *reinterpret_cast<u32x4*>(xor_ + 8 * c) = r;
+      else __builtin_nontemporal_store(r, reinterpret_cast<u32x4*>(xor_ + 8 * c));
     }
     return r;
   };
@@ -65,7 +73,7 @@ __global__ void __launch_bounds__(256) rms_norm_modulate_kernel(const uint16_t* 
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const int c = tid + 256 * i;
-    keep[i] = c < nc ? row_chunk(c) : u32x4{};
+    keep[i] = c < nc ? row_chunk(c, false) : u32x4{};
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const float a = bf16lo(keep[i][d]), b = bf16hi(keep[i][d]);
@@ -74,7 +82,7 @@ __global__ void __launch_bounds__(256) rms_norm_modulate_kernel(const uint16_t* 
     }
   }
   for (int c = tid + 256 * NR; c < nc; c += 256) {
-    const u32x4 v = row_chunk(c);
+    const u32x4 v = row_chunk(c, true);
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const float a = bf16lo(v[d]), b = bf16hi(v[d]);
@@ -96,7 +104,7 @@ __global__ void __launch_bounds__(256) rms_norm_modulate_kernel(const uint16_t* 
       const float n1 = round_bf16(bf16hi(v[d]) * r * bf16hi(wv[d]));
       o[d] = pack_bf16x2(n0 + bf16lo(sv[d]), n1 + bf16hi(sv[d]));
     }
-    *reinterpret_cast<u32x4*>(yr + 8 * c) = o;
+    __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(yr + 8 * c));
   };
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
@@ -175,19 +183,28 @@ __global__ void __launch_bounds__(256) head_rms_rope_vec_kernel(const uint16_t* 
 
 }  // namespace
 
+// rows of up to 4 * 256 chunks (H <= 8192) stay in registers between the passes
+template <bool RES, class... A>
+static hipError_t launch_rows(int T, int H, hipStream_t st, A... a) {
+  switch ((H / 8 + 255) / 256) {
+    case 1: rms_norm_modulate_kernel<1, RES><<<T, 256, 0, st>>>(a...); break;
+    case 2: rms_norm_modulate_kernel<2, RES><<<T, 256, 0, st>>>(a...); break;
+    case 3: rms_norm_modulate_kernel<3, RES><<<T, 256, 0, st>>>(a...); break;
+    default: rms_norm_modulate_kernel<4, RES><<<T, 256, 0, st>>>(a...);
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_rms_norm_modulate(const uint16_t* x, long ldx, const uint16_t* w, const uint16_t* shift, int T,
                                     int H, float eps, uint16_t* y, long ldy, hipStream_t st) {
-  // rows of up to 4 * 256 chunks (H <= 8192) stay in registers between the passes
-  rms_norm_modulate_kernel<4><<<T, 256, 0, st>>>(x, ldx, w, shift, H, eps, y, ldy);
-  return hipGetLastError();
+  return launch_rows<false>(T, H, st, x, ldx, w, shift, H, eps, y, ldy, nullptr, 0L, nullptr, nullptr, 0L);
 }
 
 hipError_t launch_residual_rms_norm_modulate(const uint16_t* x, long ldx, const uint16_t* v, long ldv,
                                              const uint16_t* g, const uint16_t* w, const uint16_t* shift, int T, int H,
                                              float eps, uint16_t* xo, long ldxo, uint16_t* y, long ldy,
                                              hipStream_t st) {
-  rms_norm_modulate_kernel<4, true><<<T, 256, 0, st>>>(x, ldx, w, shift, H, eps, y, ldy, v, ldv, g, xo, ldxo);
-  return hipGetLastError();
+  return launch_rows<true>(T, H, st, x, ldx, w, shift, H, eps, y, ldy, v, ldv, g, xo, ldxo);
 }
 
 hipError_t launch_head_rms_rope(const uint16_t* t, int T, int heads, const uint16_t* cs, const uint16_t* sn,

@@ -103,3 +103,10 @@ def test_residual_rms_norm_modulate(dev, t, h, ld):
     assert bool((diff <= _ulp(ref)).all()), "residual beyond one bf16 ulp of torch.addcmul"
     assert float((xo == ref).float().mean()) > 0.999
     assert torch.equal(y, ops.rms_norm_modulate(xo, w, shift, 1e-6))
+
+
+# rows of 1, 2, 3 and 4 chunks per thread: the last width of each kernel and the first of the next
+@pytest.mark.parametrize("h", [2048, 2056, 4096, 4104, 6152, 8192])
+def test_row_widths_at_kernel_edges(dev, h):
+    test_rms_norm_modulate_matches_torch(dev, 67, h, h + 8)
+    test_residual_rms_norm_modulate(dev, 67, h, h + 8)
