@@ -137,6 +137,12 @@ typedef struct svdq_act_sibling {
 int svdq_act_quant_siblings(const void* x, int64_t ldx, const svdq_act_sibling* layers, int count, int M, int K,
                             int group, int RTp, unsigned flags, int splits, hipStream_t stream);
 
+/* The same for the W4A16 path: layers[i].qa receives the layer's x_hat [M, K] (bf16, svdq_act_quant with
+ * SVDQ_ACT_XHAT, exact: and SVDQ_ACT_EXACT_DIV; sx is not used).  Group 64 or 128 and ranks of one, or of
+ * two, 32-column tiles run as one launch and one finalize; otherwise svdq_act_quant per layer. */
+int svdq_act_xhat_siblings(const void* x, int64_t ldx, const svdq_act_sibling* layers, int count, int M, int K,
+                           int group, int RTp, int exact, int splits, hipStream_t stream);
+
 /* Largest split-partial buffer of svdq_act_quant_noalloc, in floats (16 MiB): S * M * RTp must
  * not exceed it (S from svdq_act_quant_workspace). */
 #define SVDQ_ACT_NOALLOC_MAX_FLOATS (4 << 20)

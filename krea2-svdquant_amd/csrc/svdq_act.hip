@@ -397,6 +397,12 @@ __global__ void __launch_bounds__(256) act_siblings_kernel(ActSiblings s) {
   act_tile<G, 1, 3, false, false, false>(&s.layer[blockIdx.z]);
 }
 
+// The x_hat passes of sibling layers in one launch, likewise.
+template <int NT>
+__global__ void __launch_bounds__(256) xhat_siblings_kernel(ActSiblings s) {
+  act_tile<64, NT, 0, true, false, false>(&s.layer[blockIdx.z]);
+}
+
 // The same passes with x read once: each workgroup runs all NL layers of its row block and split.
 template <int G, int NL>
 __global__ void __launch_bounds__(256) act_shared_x_kernel(ActSiblings s) {
@@ -569,6 +575,13 @@ hipError_t launch_act(const ActParams& p, int G, int nt, int oper, bool xhat, in
   return hipErrorInvalidValue;
 }
 
+static hipError_t launch_finalize_siblings(const ActSiblings& s, int splits, hipStream_t st) {
+  const long n = (long)s.layer[0].M * (s.layer[0].RTp / 4);
+  const dim3 grid((unsigned)((n + kFinalizeThreads - 1) / kFinalizeThreads), s.count);
+  mid_finalize_siblings_kernel<<<grid, kFinalizeThreads, 0, st>>>(s, splits);
+  return hipGetLastError();
+}
+
 hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStream_t st) {
   if (s.count < 1 || s.count > MAX_SIBLINGS) return hipErrorInvalidValue;
   for (int i = 0; i < s.count; ++i)
@@ -599,10 +612,24 @@ hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStrea
     else act_siblings_kernel<128><<<grid, 256, 0, st>>>(s);
   }
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  const long n = (long)s.layer[0].M * (s.layer[0].RTp / 4);
-  const dim3 grid((unsigned)((n + kFinalizeThreads - 1) / kFinalizeThreads), s.count);
-  mid_finalize_siblings_kernel<<<grid, kFinalizeThreads, 0, st>>>(s, splits);
-  return hipGetLastError();
+  return launch_finalize_siblings(s, splits, st);
+}
+
+// A pass of each layer by itself starts and ends with CUs idle and brings a finalize of its own, two short
+// launches per layer: bound by latency, so one launch for all takes every set it can (the four attention
+// inputs / ff.up and ff.gate at rank 64 with their GEMMs, group 64, us: 64 rows 72.3 -> 42.5 / 63.5 -> 52.5, 500
+// rows 141 -> 116 / 222.6 -> 213.7, 2381 rows 531 -> 505 / 982 -> 979, 4352 rows 1049 -> 1019 / 1775 -> 1767).
+hipError_t launch_xhat_siblings(const ActSiblings& s, int nt, int splits, hipStream_t st) {
+  if (s.count < 1 || s.count > MAX_SIBLINGS || nt < 1 || nt > 2) return hipErrorInvalidValue;
+  for (int i = 0; i < s.count; ++i)   // (act_tile takes a column tile past r as LoRA's)
+    if (s.layer[i].M != s.layer[0].M || s.layer[i].K != s.layer[0].K || s.layer[i].RTp != s.layer[0].RTp ||
+        (s.layer[i].r + 31) / 32 != nt || s.layer[i].rl || s.layer[i].t0 || !s.layer[i].xhat)
+      return hipErrorInvalidValue;
+  const dim3 grid((s.layer[0].M + 63) / 64, splits, s.count);
+  if (nt == 1) xhat_siblings_kernel<1><<<grid, 256, 0, st>>>(s);
+  else xhat_siblings_kernel<2><<<grid, 256, 0, st>>>(s);
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  return launch_finalize_siblings(s, splits, st);
 }
 
 hipError_t launch_mid_finalize(const float* part, int S, int M, int RTp, uint16_t* midp, hipStream_t st) {

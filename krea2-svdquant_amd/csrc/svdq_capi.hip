@@ -274,6 +274,36 @@ int svdq_act_quant_siblings(const void* x, int64_t ldx, const svdq_act_sibling* 
   return launched(svdq::launch_act_siblings(s, group, splits, stream), "act_quant_siblings");
 }
 
+int svdq_act_xhat_siblings(const void* x, int64_t ldx, const svdq_act_sibling* layers, int count, int M, int K,
+                           int group, int RTp, int exact, int splits, hipStream_t stream) {
+  if (!layers) return fail(SVDQ_ERR_ARG, "act_xhat_siblings: null layer array");
+  if (count < 1 || count > SVDQ_MAX_SIBLINGS)
+    return fail(SVDQ_ERR_ARG, "act_xhat_siblings: count=%d, must be 1..%d", count, SVDQ_MAX_SIBLINGS);
+  const unsigned flags = SVDQ_ACT_XHAT | (exact ? SVDQ_ACT_EXACT_DIV : 0u);
+  const int nt = mid_tiles(layers[0].r, 0);
+  bool one = count > 1 && fast_group(group) && nt <= 2;
+  for (int i = 0; i < count; ++i) one = one && layers[i].r >= 1 && mid_tiles(layers[i].r, 0) == nt;
+  if (one && M > 0 && K > 0 && splits != svdq::act_splits(M, K))
+    return fail(SVDQ_ERR_ARG, "act_xhat_siblings: splits=%d, workspace says %d", splits, svdq::act_splits(M, K));
+  svdq::ActSiblings s{};
+  s.count = count;
+  for (int i = 0; i < count; ++i) {
+    const svdq_act_sibling& l = layers[i];
+    if (!one) {
+      if (int e = svdq_act_quant(x, ldx, l.srs, l.l2, l.r, nullptr, 0, nullptr, M, K, group, RTp, flags, nullptr,
+                                 nullptr, nullptr, l.qa, K, l.mid, splits, stream))
+        return e;
+      continue;
+    }
+    float* part = l.mid ? l.mid + (int64_t)(M > 0 ? M : 0) * (RTp > 0 ? RTp : 0) : nullptr;
+    if (int e = act_quant_run(x, ldx, l.srs, l.l2, l.r, nullptr, 0, nullptr, M, K, group, RTp, flags, nullptr, nullptr,
+                              nullptr, l.qa, K, l.mid, part, splits, stream, &s.layer[i]))
+      return e;
+    s.head[i] = reinterpret_cast<uint16_t*>(l.mid);
+  }
+  return one ? launched(svdq::launch_xhat_siblings(s, nt, splits, stream), "act_xhat_siblings") : SVDQ_OK;
+}
+
 int svdq_act_quant_noalloc(const void* x, int64_t ldx, const float* srs, const void* l2, int r,
                            const void* lora_down, int rl, const float* lora_mult, int M, int K, int group,
                            int RTp, unsigned flags, void* qa, void* sx, void* qx, void* xhat, int64_t ldxh,

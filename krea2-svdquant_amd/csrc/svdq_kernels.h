@@ -71,6 +71,8 @@ struct ActSiblings {
   int count;
 };
 hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStream_t st);
+// The x_hat passes (no codes) of such layers, each of nt (1 or 2) rank tiles, and their finalize.
+hipError_t launch_xhat_siblings(const ActSiblings& s, int nt, int splits, hipStream_t st);
 
 int act_splits(int M, int K);
 // oper: 0 = no codes (x_hat only), 1 = e4m3 operand codes, 2 = int8 16*q operand codes, 3 = e3m2;

@@ -223,7 +223,7 @@ std::vector<Tensor> linear_siblings(const Tensor& x, const std::vector<Tensor>& 
   const c10::DeviceGuard guard(c.dev);
   Layer l[SVDQ_MAX_SIBLINGS];
   std::vector<Tensor> ys;
-  bool one_pass = operand == SVDQ_OPERAND_E3M2;   // one launch for the activation passes
+  bool one_pass = operand == SVDQ_OPERAND_E3M2 || !c.quant;   // one launch for the activation passes
   for (size_t i = 0; i < count; ++i) {
     l[i] = c.layer(srs[i], l2[i], lora_down.get(i), lora_mult.get(i), rtp[i], weight[i], weight_scales[i], l1cat[i],
                    bias.get(i));
@@ -237,10 +237,14 @@ std::vector<Tensor> linear_siblings(const Tensor& x, const std::vector<Tensor>& 
   if (one_pass) {
     svdq_act_sibling a[SVDQ_MAX_SIBLINGS];
     for (size_t i = 0; i < count; ++i)
-      a[i] = {ptr<float>(srs[i]), ptr(l2[i]), (int)l[i].r, base + l[i].qa, base + l[i].sx,
-              reinterpret_cast<float*>(base + l[i].mid)};
-    check_status("svdq_act_quant_siblings", svdq_act_quant_siblings(ptr(c.x), k, a, (int)count, m, k, (int)group,
-                                                                    (int)rtp[0], c.flags(exact), l[0].splits, st));
+      a[i] = {ptr<float>(srs[i]), ptr(l2[i]), (int)l[i].r, base + (c.quant ? l[i].qa : l[i].xhat),
+              c.quant ? base + l[i].sx : nullptr, reinterpret_cast<float*>(base + l[i].mid)};
+    if (c.quant)
+      check_status("svdq_act_quant_siblings", svdq_act_quant_siblings(ptr(c.x), k, a, (int)count, m, k, (int)group,
+                                                                      (int)rtp[0], c.flags(exact), l[0].splits, st));
+    else
+      check_status("svdq_act_xhat_siblings", svdq_act_xhat_siblings(ptr(c.x), k, a, (int)count, m, k, (int)group,
+                                                                    (int)rtp[0], exact, l[0].splits, st));
   } else {
     for (size_t i = 0; i < count; ++i) c.act_quant(l[i], base, exact, st);
   }

@@ -238,7 +238,7 @@ def forward_prepared_siblings(x: Tensor, preps: Sequence[PreparedLayer], *, mode
     """Forwards of sibling layers (same input ``x``, same K and group size) on prepared operands.
     W4A4: an activation pass per layer (each layer has its own smoothing; one launch for all when
     none has LoRA adapters, ``svdq::act_quant_siblings``), then the layers' GEMMs as one launch
-    (``svdq::w4a4_gemm_siblings``).  W4A16: each layer's x_hat pass, then the layers' GEMMs as one
+    (``svdq::w4a4_gemm_siblings``).  W4A16: the x_hat passes likewise, then the layers' GEMMs as one
     launch where that pays (``svdq::w4a16_gemm_siblings``).  Every output is bit-identical to
     ``forward_prepared(x, prep, mode=mode)`` of its layer."""
     if not x.is_cuda:

@@ -85,6 +85,7 @@ SIGNATURES = {
     "svdq_w4a16_gemm_epi": (_I, [_P, _L, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P, _L, _I,
                                  _I, _P, _L, _P, _P]),
     "svdq_act_quant_siblings": (_I, [_P, _L, ctypes.POINTER(ActSibling), _I, _I, _I, _I, _I, _U, _I, _P]),
+    "svdq_act_xhat_siblings": (_I, [_P, _L, ctypes.POINTER(ActSibling), _I, _I, _I, _I, _I, _I, _I, _P]),
     "svdq_w4a4_gemm_siblings": (_I, [ctypes.POINTER(W4A4Sibling), _I, _I, _I, _I, _I, _I, _P]),
     "svdq_w4a16_gemm_siblings": (_I, [ctypes.POINTER(W4A16Sibling), _I, _I, _I, _I, _I, _P]),
     "svdq_gate_op": (_I, [_I, _P, _P, _P, _L, _P]),
