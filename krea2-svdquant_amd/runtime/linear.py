@@ -155,10 +155,16 @@ class SVDQuantLinear(nn.Module):
         return _HIP_MODES[self.resolved_backend(device)]
 
     def _buffers_key(self, device: torch.device) -> tuple:
-        # storage and version counter of every buffer: in-place edits bump the version
+        # storage and version counter of every operand: in-place edits bump the version.  Read from
+        # _buffers where it is there (Module's attribute lookup takes 0.3 us each); an operand that
+        # was replaced by a Parameter or parametrized, and a bias set on a layer built without one
+        # (a plain attribute), live elsewhere.
         b = self._buffers
-        q, sm, ws, l1, l2, bias = (b["qweight"], b["smooth_scale"], b["weight_scales"], b["l1"], b["l2"],
-                                   b.get("bias"))
+        try:
+            q, sm, ws, l1, l2 = b["qweight"], b["smooth_scale"], b["weight_scales"], b["l1"], b["l2"]
+        except KeyError:
+            q, sm, ws, l1, l2 = self.qweight, self.smooth_scale, self.weight_scales, self.l1, self.l2
+        bias = b["bias"] if "bias" in b else self.bias
         return (device, q.data_ptr(), q._version, sm.data_ptr(), sm._version, ws.data_ptr(), ws._version,
                 l1.data_ptr(), l1._version, l2.data_ptr(), l2._version,
                 None if bias is None else (bias.data_ptr(), bias._version))

@@ -166,3 +166,34 @@ def test_checkpoint_and_lora_loaders_end_to_end(dev, tmp_path):
         e = rel_l2(y, nm.bf16(sim.w4a4_eval(x, st)["y"].astype(np.float32)))
         print(f"  loaded {tuple(st.shape)} adapters={len(adapters)} rel_l2={e:.3e}")
         assert e < 1e-3
+
+
+@pytest.mark.parametrize("backend", ["hip_gfx950", "hip_gfx950_w4a16"])
+def test_operands_replaced_after_a_forward(dev, backend):
+    """A bias set on a layer built without one, a Parameter bias edited in place and operands replaced
+    by Parameters after a forward: each output is that of a fresh layer of the new state."""
+    from krea2_svdquant_amd.runtime.linear import SVDQuantLinear
+    x = synth.make_activation(40, 256, seed=51)
+    mod = SVDQuantLinear(to_device_state(synth.make_layer(72, 256, x, rank=32, group_size=64, seed=52), dev),
+                         backend=backend)
+    xd = bf16_tensor(x, dev)
+    outs = [mod(xd)]
+
+    def check():
+        y = mod(xd)
+        assert torch.equal(y, SVDQuantLinear(mod.state, backend=backend)(xd))
+        assert not torch.equal(y, outs[-1])
+        outs.append(y)
+
+    with torch.no_grad():
+        mod.bias = torch.ones(72, dtype=torch.bfloat16, device=dev)
+        check()
+        mod.bias = torch.nn.Parameter(torch.full((72,), 2.0, dtype=torch.bfloat16, device=dev))
+        check()
+        mod.bias.mul_(2)
+        check()
+        for name in ("l1", "l2", "smooth_scale", "weight_scales"):
+            setattr(mod, name, torch.nn.Parameter(getattr(mod, name) * 2))
+            check()
+            getattr(mod, name).mul_(0.5)
+            check()

@@ -4,6 +4,7 @@ instead of any fallback."""
 import numpy as np
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 from krea2_svdquant_amd import BACKEND_CHOICES, BackendKind, SVDQuantConfig, SVDQuantLinearState
 from krea2_svdquant_amd.quant import convert
@@ -151,3 +152,39 @@ def test_backend_function_caches_prepared_operands_per_state(monkeypatch):
     del st
     gc.collect()
     assert key not in backend._SEAM_CACHE
+
+
+def test_operand_key_sees_every_attribute():
+    """The key of the cached kernel operands follows what ``state`` returns: buffers, Parameters that
+    replaced them, parametrized buffers, and a bias set on a layer built without one."""
+    dev = torch.device("cpu")
+    for name in ("qweight", "smooth_scale", "weight_scales", "l1", "l2"):
+        mod = SVDQuantLinear(_state(), backend="hip_gfx950")
+        keys = [mod._buffers_key(dev)]
+        setattr(mod, name, torch.nn.Parameter(getattr(mod, name).clone(), requires_grad=False))
+        keys.append(mod._buffers_key(dev))
+        with torch.no_grad():
+            getattr(mod, name).zero_()
+        keys.append(mod._buffers_key(dev))
+        assert len(set(keys)) == 3, name
+    mod = SVDQuantLinear(_state(), backend="hip_gfx950")
+    keys = [mod._buffers_key(dev)]
+    mod.bias = torch.zeros(3, dtype=torch.bfloat16)
+    keys.append(mod._buffers_key(dev))
+    mod.bias.add_(1)
+    keys.append(mod._buffers_key(dev))
+    mod.bias = torch.nn.Parameter(torch.zeros(3, dtype=torch.bfloat16))
+    keys.append(mod._buffers_key(dev))
+    with torch.no_grad():
+        mod.bias.add_(1)
+    keys.append(mod._buffers_key(dev))
+    mod.bias = None
+    assert len(set(keys)) == 5 and mod._buffers_key(dev) == keys[0]
+
+    class Doubled(torch.nn.Module):
+        def forward(self, t):
+            return 2 * t
+
+    before = mod._buffers_key(dev)
+    torch.nn.utils.parametrize.register_parametrization(mod, "l1", Doubled())
+    assert mod._buffers_key(dev) != before
