@@ -101,12 +101,12 @@ __device__ __forceinline__ void mfma_out(f32x16& acc, u32x4 a, u32x4 b) {
 // items that fill whole rounds over the CUs run one workgroup each; the rest (a last, partly
 // filled round) are cut into `split` pieces along the keys -- `per` key tiles each -- whose
 // partial outputs attn_combine_kernel merges, so that the last round takes about 1 / split of
-// a full item's time.  Merging costs a launch and the float32 partials' way through memory, the
-// time of about four key tiles, so items whose pieces would save fewer stay whole, and so do items
-// that leave no room for two pieces.  48 heads, us per call, in pieces / whole: T = 64 (one piece) 14.8 /
-// 9.6, T = 128 (2 pieces, 1 tile saved) 17.1 / 13.1, T = 384 (2, 3) 25.1 / 23.9, T = 512 (2, 4) 27.2 / 27.7,
-// T = 1101 (one piece) 56.1 / 48.0, T = 1500 (8, 21) 87 / 112, T = 2381 (one piece) 175.6 / 168.2.
-constexpr int MERGE_TILES = 4;   // key tiles that merging an item's pieces costs
+// a full item's time.  Items that leave no room for two pieces stay whole: a piece that holds all
+// keys gives the same output and a merge that does nothing (48 heads, us per call, in one piece / whole:
+// T = 64 14.8 / 9.6, T = 1101 56.1 / 48.0, T = 2381 175.6 / 168.2).  Two pieces that save less than
+// the merge costs, about four key tiles, are kept (T = 128 17.1 / 13.1, T = 384 25.1 / 23.9): their
+// outputs are nearer to 64 bits than a whole item's (relative error 2.188e-3 / 2.251e-3 and 2.289e-3 /
+// 2.313e-3, each piece's probabilities being rounded against an offset of its own).
 struct AttnPlan {
   int nq, items, nmain, tail, split, per;
 };
@@ -121,7 +121,7 @@ __host__ __device__ inline AttnPlan attn_plan(int T, int H, int cus) {
   split = split < 1 ? 1 : split > 8 ? 8 : split > nt ? nt : split;
   pl.per = (nt + split - 1) / split;
   pl.split = (nt + pl.per - 1) / pl.per;   // no empty piece
-  if (nt - pl.per < MERGE_TILES) {
+  if (pl.split == 1) {
     pl.nmain = pl.items;
     pl.tail = 0;
   }

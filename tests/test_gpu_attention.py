@@ -131,10 +131,10 @@ def test_attention_scores_far_above_the_first_keys(dev):
 
 
 def test_attention_tail_pieces_hand_over_overflowing_products(dev):
-    """T=300 at 48 query heads: 96 items, all in the last, partly filled round and kept whole (512
-    tokens, cut into key pieces: ``test_gpu_attention_rounds.py``).  Keys 32.. score 56 log2 units above the first 32
+    """T=300 at 48 query heads: 96 items, all in the last, partly filled round, so every item runs
+    as key pieces merged by the combine kernel.  Keys 32.. score 56 log2 units above the first 32
     keys (the fixed exponent offset), so a probability reaches 2^56 while the row sum stays below
-    2^64, and every v is 2^73: p v passes the f32 range.  Those waves must hand
+    2^64, and every v is 2^73: p v passes the f32 range in the first piece.  Those waves must hand
     their queries to the running-maximum kernel (as whole items do through their normalized
     output), and the output is the average of equal values, 2^73, exactly."""
     t, heads, kvh = 300, 48, 12

@@ -1,5 +1,5 @@
-"""GPU tests of the attention's last round of workgroups: items cut into key pieces where the pieces
-save at least four key tiles, whole items otherwise (``svdq_attn.hip``, ``attn_plan``).
+"""GPU tests of the attention's last round of workgroups: items cut into key pieces where there is
+room for two of each, whole items otherwise (``svdq_attn.hip``, ``attn_plan``).
 
 The workspace tells which it is: 16 bytes of flags per item, and more than that only with pieces.
 48 query heads over 256-query items; tolerance as in ``test_gpu_attention.py``.
@@ -22,9 +22,9 @@ def _in_pieces(t, heads):
 @pytest.mark.parametrize("t,pieces", [
     (1, False),       # a single key
     (64, False),      # one key tile: nothing to cut
-    (65, False),      # two pieces would save one tile
-    (448, False),     # 7 tiles in two pieces: 3 saved
-    (449, True),      # 8 tiles in two pieces: 4 saved
+    (65, True),       # two pieces, the second of one key
+    (448, True),      # 7 tiles in two pieces
+    (449, True),
     (512, True),
     (513, False),     # 144 items: no room for two pieces
     (1279, False),    # 240 items, a partial key tile and query block
@@ -36,7 +36,7 @@ def test_last_round_matches_float32(dev, t, pieces):
     _check(*_inputs(t, 48, 12, dev, seed=t))
 
 
-@pytest.mark.parametrize("t,pieces", [(300, False), (512, True)])
+@pytest.mark.parametrize("t,pieces", [(64, False), (300, True), (512, True), (700, False)])
 def test_overflowing_products_hand_over(dev, t, pieces):
     """Keys 32.. score 56 log2 units above the first 32 (the fixed exponent offset) and every v is
     2^73: p v passes the f32 range while the row sum stays below 2^64.  The waves hand over to the
