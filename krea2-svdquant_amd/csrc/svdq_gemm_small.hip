@@ -5,6 +5,7 @@
 // MFMA, S = sx (x) sw on the bf16 MFMA, acc += P * S in group order, then mid @ l1cat^T (hi plane,
 // lo plane, 16 ranks at a time) and the bias.  Every output therefore has the same bits on every
 // tile, and the choice of tile is free.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -367,6 +368,7 @@ constexpr SmallTile kSmallTiles[] = {
 };
 constexpr int kSmallCount = sizeof(kSmallTiles) / sizeof(kSmallTiles[0]);
 constexpr int kCUs = 256;
+constexpr int kMaxRows = 1 << 25;
 
 long tile_count(int M, const int* N, int count, int tm, int tn) {
   long t = 0;
@@ -407,6 +409,9 @@ int w4a4_small_tile(int M, const int* N, int count, int K, int G) {
       if (!strcmp(e, kSmallTiles[t].name)) return t;
     if (!strcmp(e, "256x128") || !strcmp(e, "256x256")) return -1;
   }
+  // a lane's offset within a stage spans 8 planes of 16 bytes per row, in 32 bits
+  for (int i = 0; i < count; ++i)
+    if (std::max(M, N[i]) > kMaxRows) return -1;
   const long large = tile_count(M, N, count, 256, 128);
   const long whole = large / kCUs, part = large % kCUs;
   float best = 0.95f * (52.0f * whole + (part ? 42.0f + 10.0f * part / kCUs : 0.0f));
@@ -426,7 +431,8 @@ hipError_t launch_w4a4_small(const GemmSiblings& gs, int G, int tile, bool out_f
   long tiles = 0;
   for (int i = 0; i < w.count; ++i) {
     const GemmParams& p = w.layer[i];
-    if (p.M != w.layer[0].M || p.K != w.layer[0].K || p.K % G || p.epi || p.RTp % 32) return hipErrorInvalidValue;
+    if (p.M != w.layer[0].M || p.K != w.layer[0].K || p.K % G || p.epi || p.RTp % 32 || std::max(p.M, p.N) > kMaxRows)
+      return hipErrorInvalidValue;
     w.tile0[i] = (int)tiles;
     tiles += tile_count(p.M, &p.N, 1, kSmallTiles[tile].tm, kSmallTiles[tile].tn);
     if (tiles > 0x7FFFFFFF) return hipErrorInvalidValue;

@@ -245,3 +245,12 @@ def test_w4a4_tile_choice():
             os.environ.pop("SVDQ_W4A4_TILES", None)
         else:
             os.environ["SVDQ_W4A4_TILES"] = old
+
+
+def test_w4a4_small_tiles_keep_32_bit_offsets():
+    """The small tiles address a stage's eight 16-byte planes by 32-bit offsets: up to 2^25 rows or
+    columns; wider operands take the 256-row tiles, whose plane bases are 64 bits."""
+    t = lib.w4a4_tile_cols
+    assert t(64, 1536, 6144, 64, 2) == 0 and t(1 << 25, 32, 64, 64, 2) in (0, 128)
+    assert t((1 << 25) + 2, 32, 64, 64, 2) == 128 and t(32, (1 << 25) + 2, 64, 64, 2) == 128
+    assert t(16, (1 << 25) + 2, 128, 128, 2) == 128
