@@ -144,7 +144,8 @@ int svdq_act_xhat_siblings(const void* x, int64_t ldx, const svdq_act_sibling* l
                            int group, int RTp, int exact, int splits, hipStream_t stream);
 
 /* Largest split-partial buffer of svdq_act_quant_noalloc, in floats (16 MiB): S * M * RTp must
- * not exceed it (S from svdq_act_quant_workspace). */
+ * not exceed it (S from svdq_act_quant_workspace, or with group 128 at most max(1, K / 512) where
+ * that S does not fit: the low-rank activations are then summed over fewer, longer partials). */
 #define SVDQ_ACT_NOALLOC_MAX_FLOATS (4 << 20)
 
 /* svdq_act_quant without any allocation or caller workspace.  No counterpart in the reference:

@@ -557,12 +557,12 @@ hipError_t launch_act_g(const ActParams& p, int nt, int oper, bool xhat, dim3 gr
 
 }  // namespace
 
-int act_splits(int M, int K) {
+int act_splits(int M, int K, int cols) {
   // 512 workgroups fill the 256 CUs once (two 4-wave workgroups per CU): as many K splits as keep
   // row_tiles * splits within that, so no workgroups are left over for a second round
   const int row_tiles = (M + 63) / 64;
   int s = 512 / row_tiles;
-  const int smax = K / 256 > 0 ? K / 256 : 1;   // 64 columns for each of a workgroup's waves
+  const int smax = K / cols > 0 ? K / cols : 1;
   if (s > smax) s = smax;
   if (s < 1) s = 1;
   return s;

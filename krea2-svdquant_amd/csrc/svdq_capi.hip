@@ -311,7 +311,9 @@ int svdq_act_quant_noalloc(const void* x, int64_t ldx, const float* srs, const v
   if (M <= 0) return fail(SVDQ_ERR_ARG, "act_quant_noalloc: M=%d", M);
   if (int e = check_group(group, K)) return e;
   if (RTp <= 0 || RTp % 32) return fail(SVDQ_ERR_SHAPE, "act_quant_noalloc: RTp=%d must be a positive multiple of 32", RTp);
-  const int splits = svdq::act_splits(M, K);
+  int splits = svdq::act_splits(M, K);
+  // group 128: whole groups for each of a workgroup's waves where the partials of more splits do not fit
+  if (group == 128 && (int64_t)splits * M * RTp > kScratchFloats) splits = svdq::act_splits(M, K, 512);
   const int64_t need = (int64_t)splits * M * RTp;
   if (need > kScratchFloats)
     return fail(SVDQ_ERR_SHAPE,

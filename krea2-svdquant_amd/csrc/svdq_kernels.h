@@ -74,7 +74,8 @@ hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStrea
 // The x_hat passes (no codes) of such layers, each of nt (1 or 2) rank tiles, and their finalize.
 hipError_t launch_xhat_siblings(const ActSiblings& s, int nt, int splits, hipStream_t st);
 
-int act_splits(int M, int K);
+// K splits of the pass over M rows, each of at least cols columns (256: 64 for each of a workgroup's waves)
+int act_splits(int M, int K, int cols = 256);
 // oper: 0 = no codes (x_hat only), 1 = e4m3 operand codes, 2 = int8 16*q operand codes, 3 = e3m2;
 // nt: column tiles of the down projections from p.t0 (at most 4); with p.t0 > 0 the launch computes
 // down projections only (oper 0, no x_hat); launches without codes take G = 64

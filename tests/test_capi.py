@@ -254,3 +254,22 @@ def test_w4a4_small_tiles_keep_32_bit_offsets():
     assert t(64, 1536, 6144, 64, 2) == 0 and t(1 << 25, 32, 64, 64, 2) in (0, 128)
     assert t((1 << 25) + 2, 32, 64, 64, 2) == 128 and t(32, (1 << 25) + 2, 64, 64, 2) == 128
     assert t(16, (1 << 25) + 2, 128, 128, 2) == 128
+
+
+@pytest.mark.parametrize("m,k,g,rtp,fits", [
+    (1024, 6144, 128, 160, True),     # 24 splits fit
+    (1024, 6144, 128, 192, True),     # 24 x 1024 x 192 floats do not, 12 splits do
+    (1024, 6144, 128, 320, True),
+    (1024, 6144, 128, 352, False),
+    (500, 16384, 128, 160, True),
+    (1024, 6144, 64, 192, False),     # group 64: always splits of 256 columns
+    (64, 128, 128, 32, True),
+])
+def test_act_quant_noalloc_scratch_limit(m, k, g, rtp, fits):
+    """Which calls the scratch admits: one that is refused names the scratch, one that fits is refused
+    for what follows that check (here a null activation pointer)."""
+    fake = ctypes.c_void_p(0x1000)
+    with pytest.raises(lib.SVDQError) as ei:
+        lib.call("svdq_act_quant_noalloc", None, k, fake, fake, 32, None, 0, None, m, k, g, rtp,
+                 lib.SVDQ_ACT_OPERAND_E3M2 | lib.SVDQ_ACT_SX_PAIRS, fake, fake, None, None, k, fake, None)
+    assert ("device scratch" in str(ei.value)) == (not fits)

@@ -86,3 +86,33 @@ def test_noalloc_config1_ffup_rows(dev):
     st = synth.make_layer(512, 6144, x[:256], rank=32, group_size=64, seed=72)
     prep = backend.prepare_layer(to_device_state(st, dev), (), dev)
     _call_pair(dev, bf16_tensor(x, dev), prep, st, 64)
+
+
+def test_noalloc_group128_with_fewer_splits(dev):
+    """M = 1024, K = 6144, group 128, ranks 128 + 64: the workspace entry point's 24 splits do not fit
+    the scratch, so the partials are those of 12.  Codes and scales are the same bits; the low-rank
+    activations are sums of K products in another order, within K 2^-24 of the sum of magnitudes (and
+    2^-16 for the two bf16 planes)."""
+    from krea2_svdquant_amd.kernels.hip import lib, ops
+    m, k, g, r, rl = 1024, 6144, 128, 128, 64
+    gen = torch.Generator(device=dev).manual_seed(81)
+    x = torch.randn(m, k, device=dev, generator=gen).to(torch.bfloat16)
+    s = (torch.rand(k, device=dev, generator=gen) + 0.5).to(torch.bfloat16)
+    srs = ops.prepare_smooth(s)
+    l2 = (torch.randn(r, k, device=dev, generator=gen) * 0.05).to(torch.bfloat16)
+    down = (torch.randn(rl, k, device=dev, generator=gen) * 0.05).to(torch.bfloat16)
+    mult = torch.full((rl,), 0.5, device=dev)
+    rtp = ops.rank_padded(r + rl)
+    qa, sx, _, _, mid = ops.act_quant(x, srs, l2, down, mult, g, rtp, ops.OPERAND_E3M2, False, False, False, True)
+    assert (mid.shape[0] - 1) * m * rtp > lib.SVDQ_ACT_NOALLOC_MAX_FLOATS
+    qa1, sx1 = torch.empty_like(qa), torch.empty_like(sx)
+    head = torch.empty((1, m, rtp), dtype=torch.float32, device=dev)
+    lib.call("svdq_act_quant_noalloc", _vp(x), k, _vp(srs), _vp(l2), r, _vp(down), rl, _vp(mult), m, k, g, rtp,
+             lib.SVDQ_ACT_OPERAND_E3M2 | lib.SVDQ_ACT_SX_PAIRS, _vp(qa1), _vp(sx1), None, None, k, _vp(head),
+             ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream))
+    assert torch.equal(qa, qa1) and torch.equal(sx, sx1)
+    xh = (x.float() / s.float()).to(torch.bfloat16).double()
+    want = torch.cat((xh @ l2.double().T, 0.5 * (x.double() @ down.double().T)), 1)
+    mag = torch.cat((xh.abs() @ l2.double().abs().T, 0.5 * (x.double().abs() @ down.double().abs().T)), 1)
+    for v in (mid, head):
+        assert bool(((ops.mid_values(v).double() - want).abs() <= mag * (k * 2.0 ** -24 + 2.0 ** -16)).all())
