@@ -64,7 +64,7 @@ def torch_command(out: Path) -> list[str]:
     root = Path(torch.__file__).resolve().parent
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     return [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall",
-            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DSVDQ_TORCH_BUILD="{torch.__version__}"', "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
             "-isystem", str(root / "include"), "-isystem", str(root / "include/torch/csrc/api/include"),
             "-isystem", f"{rocm}/include", str(CSRC / "svdq_torch.cpp"), "-L", str(root / "lib"), "-lc10", "-lc10_hip",
             "-ltorch_cpu", "-o", str(out)]

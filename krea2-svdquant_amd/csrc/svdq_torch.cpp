@@ -267,6 +267,10 @@ std::vector<Tensor> linear_siblings(const Tensor& x, const std::vector<Tensor>& 
 
 }  // namespace
 
+// The torch that this file was compiled against, found in the file by kernels/hip/lib.py ahead of
+// loading it: the C++ interfaces used here hold for that build of torch only.
+extern "C" __attribute__((used, visibility("default"))) const char svdq_torch_build[] = "svdq_torch built with torch " SVDQ_TORCH_BUILD;
+
 TORCH_LIBRARY_FRAGMENT(svdq, m) {
   m.def(
       "linear(Tensor x, Tensor srs, Tensor l2, Tensor? lora_down, Tensor? lora_mult, int group_size, int rtp, "

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import re
 import threading
 from pathlib import Path
 
@@ -137,6 +138,10 @@ def load_torch_ops() -> None:
     load()
     if not TORCH_LIB_PATH.exists():
         raise RuntimeError(f"torch operators not found at {TORCH_LIB_PATH}; build them with __graft_entry__.build()")
+    built = re.search(rb"svdq_torch built with torch ([^\0]*)\0", TORCH_LIB_PATH.read_bytes())
+    if built is None or built.group(1).decode() != torch.__version__:
+        raise RuntimeError(f"{TORCH_LIB_PATH} was built with torch {built.group(1).decode() if built else 'unknown'}, "
+                           f"this process runs torch {torch.__version__}; build it again with __graft_entry__.build()")
     torch.ops.load_library(str(TORCH_LIB_PATH))
 
 

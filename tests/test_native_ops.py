@@ -82,3 +82,18 @@ def test_refusals(dev):
     x = torch.randn(4, 256, device=dev).to(torch.bfloat16).requires_grad_()
     with pytest.raises(RuntimeError):
         forward_prepared(x, p).sum().backward()
+
+
+@pytest.mark.skipif(not lib.TORCH_LIB_PATH.exists(), reason="library not built")
+def test_operators_of_another_torch_are_refused_before_loading(tmp_path, monkeypatch):
+    mark = b"svdq_torch built with torch "
+    data = lib.TORCH_LIB_PATH.read_bytes()
+    assert mark + torch.__version__.encode() + b"\0" in data
+    other = tmp_path / "libsvdq_torch.so"
+    monkeypatch.setattr(lib, "TORCH_LIB_PATH", other)
+    monkeypatch.setattr(torch.ops, "load_library", lambda path: pytest.fail("loaded"))
+    for content, needle in ((data.replace(mark + torch.__version__[:1].encode(), mark + b"0"), "built with torch 0"),
+                            (data.replace(mark, b"x" * len(mark)), "built with torch unknown")):
+        other.write_bytes(content)
+        with pytest.raises(RuntimeError, match=needle):
+            lib.load_torch_ops()
