@@ -278,12 +278,11 @@ int svdq_w4a4_gemm_siblings(const svdq_w4a4_sibling* layers, int count, int oper
  * M, K and group; each layer with its own x_hat from its own svdq_act_quant, since the smoothing
  * differs per layer), e.g. attn.to_q / to_gate / to_k / to_v.  The reference calls them one after
  * another through SVDQuantLinear.forward (reference runtime/linear.py:156-161); each output here
- * equals svdq_w4a16_gemm's for that layer bit for bit.  With group 64 or 128 and every layer fit
- * for the specialized-wave kernel (no fused op; x_hat 16-byte aligned rows) the layers' 192 x 256
- * output tiles run in one launch when their rounds over the CUs cost no more than the layers'
- * own launches (the attention inputs at M = 2304: 720 tiles in 3 rounds against 2 rounds of
- * 256 x 256 tiles and 2 of 128 x 128 tiles); otherwise the layers run one after another on
- * `stream`.
+ * equals svdq_w4a16_gemm's for that layer bit for bit.  With group 64 or 128 the layers' output
+ * tiles run in one launch, of the tile that takes least by its rounds over the CUs, where that costs
+ * no more than the layers' own launches (the attention inputs at M = 4352: 8 rounds of 128 x 256 tiles, 736 us by the
+ * rule, against 904 in four launches); otherwise the layers run one after another on
+ * `stream`.  svdq_w4a16_gemm_tile tells which it is.
  *   layers[i]: the per-layer arguments of svdq_w4a16_gemm, with out_f32 = 0 or 1 for all. */
 typedef struct svdq_w4a16_sibling {
   const void* xhat;
@@ -300,6 +299,13 @@ typedef struct svdq_w4a16_sibling {
 } svdq_w4a16_sibling;
 int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M, int K, int group, int out_f32,
                              hipStream_t stream);
+
+/* Block tile (*rows x *cols, either may be null) that svdq_w4a16_gemm (count 1) or
+ * svdq_w4a16_gemm_siblings (N[i] columns of layer i) runs over M contiguous rows of x_hat, group 64 or
+ * 128, RTp as in those calls, no fused op; returns the number of launches: 1, or count where each
+ * layer runs by itself (the tile is then the first layer's), 0 for other arguments.  No reference
+ * counterpart: a host-side query for callers that report which kernel ran (tests). */
+int svdq_w4a16_gemm_tile(int M, const int* N, int count, int K, int group, int RTp, int* rows, int* cols);
 
 /* The sigmoid output gate and the SwiGLU product of a DiT block as one pass each over contiguous
  * bf16 tensors: out[i] = op(y[i], aux[i]) with op SVDQ_EPI_MUL_SIGMOID (aux * sigmoid(y)) or

@@ -625,6 +625,41 @@ int svdq_w4a16_gemm_epi(const void* xhat, int64_t ldxh, const void* qw, const vo
   return launched(svdq::launch_w4a16(p, group, out_f32 == 1, stream), "w4a16_gemm");
 }
 
+// The launch that takes all the layers, or false where a launch per layer costs less or does not exist.
+static bool w4a16_grouped(const svdq::GemmSiblings& gs, int group, svdq::W4A16Route& r) {
+  r = svdq::w4a16_route(gs);
+  long own = 0;   // cost of a launch per layer
+  for (int i = 0; i < gs.count; ++i) {
+    svdq::GemmSiblings one{};
+    one.count = 1;
+    one.layer[0] = gs.layer[i];
+    own += svdq::w4a16_route(one).cost;
+  }
+  return fast_group(group) && r.tile != svdq::W4A16_WIDE && r.cost <= own;
+}
+
+int svdq_w4a16_gemm_tile(int M, const int* N, int count, int K, int group, int RTp, int* rows, int* cols) {
+  if (!N || count < 1 || count > SVDQ_MAX_SIBLINGS || M <= 0 || K <= 0 || !fast_group(group) || K % group || RTp <= 0 ||
+      RTp % 32)
+    return 0;
+  svdq::GemmSiblings gs{};
+  gs.count = count;
+  for (int i = 0; i < count; ++i) {
+    if (N[i] <= 0) return 0;
+    gs.layer[i] = gemm_params(nullptr, nullptr, nullptr, nullptr, RTp, nullptr, M, N[i], K, nullptr, N[i]);
+    gs.layer[i].ldxh = K;
+  }
+  svdq::W4A16Route r;
+  const int launches = w4a16_grouped(gs, group, r) ? 1 : count;
+  gs.count = 1;
+  if (launches > 1) r = svdq::w4a16_route(gs);
+  int tm, tn;
+  svdq::w4a16_tile(r.tile, tm, tn);
+  if (rows) *rows = tm;
+  if (cols) *cols = tn;
+  return launches;
+}
+
 int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M, int K, int group, int out_f32,
                              hipStream_t stream) {
   if (!layers) return fail(SVDQ_ERR_ARG, "w4a16_gemm_siblings: null layer array");
@@ -633,7 +668,6 @@ int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M,
   svdq::GemmSiblings gs{};
   gs.count = count;
   int tiles = 0;
-  long own = 0;   // cost of a launch per layer
   for (int i = 0; i < count; ++i) {
     const svdq_w4a16_sibling& l = layers[i];
     if (int e = gemm_common_checks("w4a16_gemm_siblings", l.qw, l.sw, l.mid, l.l1cat, l.RTp, M, l.N, K, group, l.y,
@@ -647,15 +681,11 @@ int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M,
     p = gemm_params(l.qw, l.sw, l.mid, l.l1cat, l.RTp, l.bias, M, l.N, K, l.y, l.ldy);
     p.xhat = static_cast<const uint16_t*>(l.xhat);
     p.ldxh = l.ldxh;
-    svdq::GemmSiblings one{};
-    one.count = 1;
-    one.layer[0] = p;
-    own += svdq::w4a16_route(one).cost;
     gs.tile0[i] = tiles;
     tiles += ((M + 191) / 192) * ((l.N + 255) / 256);
   }
   gs.tile0[count] = tiles;
-  if (const svdq::W4A16Route r = svdq::w4a16_route(gs); fast_group(group) && r.tile != svdq::W4A16_WIDE && r.cost <= own)
+  if (svdq::W4A16Route r; w4a16_grouped(gs, group, r))
     return launched(r.tile == svdq::W4A16_WS ? svdq::launch_w4a16_siblings(gs, group, out_f32 == 1, stream)
                                              : svdq::launch_w4a16_direct(gs, group, r.tile, out_f32 == 1, stream),
                     "w4a16_gemm_siblings");

@@ -117,6 +117,7 @@ struct W4A16Route {
   long cost;
 };
 W4A16Route w4a16_route(const GemmSiblings& gs);
+void w4a16_tile(int tile, int& rows, int& cols);   // its block tile
 hipError_t launch_w4a16_direct(const GemmSiblings& gs, int G, int tile, bool out_f32, hipStream_t st);
 // Sibling layers (tile0 in 192 x 256 tiles, filled in by the caller) in one launch of the
 // specialized-wave kernel; hipErrorInvalidValue when a layer cannot take it (w4a16_ws_fits).

@@ -5,6 +5,7 @@
 // Same operands, arithmetic and order as the tiles that stage the dequantized weights through LDS
 // (svdq_gemm.hip): 16 columns of K per bf16 MFMA in order, then hi and lo low-rank products 16 ranks at
 // a time, bias, one rounding.  Every output has the same bits on every kernel.
+#include <climits>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -379,8 +380,9 @@ W4A16Route w4a16_route(const GemmSiblings& gs) {
     for (int i = 0; i < gs.count; ++i) t += ((long)gs.layer[i].M + tm - 1) / tm * (((long)gs.layer[i].N + tn - 1) / tn);
     return (t + 255) / 256;
   };
-  W4A16Route best{W4A16_WIDE, kWideCost * rounds(256, 256)};
-  if (gs.count > 1 && ke && !strcmp(ke, "wide")) return best;   // each layer by its own rule
+  // (sibling layers have no launch of 256 x 256 tiles: WIDE then means each layer by its own rule)
+  W4A16Route best{W4A16_WIDE, gs.count > 1 ? LONG_MAX : kWideCost * rounds(256, 256)};
+  if (gs.count > 1 && ke && !strcmp(ke, "wide")) return best;
   if (ws && kWsCost * rounds(192, 256) <= best.cost) best = {W4A16_WS, kWsCost * rounds(192, 256)};
   for (int t = 0; t < kTileCount && direct; ++t) {
     if (e && !strcmp(e, kTiles[t].name)) return {t, 0};
@@ -388,6 +390,11 @@ W4A16Route w4a16_route(const GemmSiblings& gs) {
     if (c < best.cost) best = {t, c};
   }
   return best;
+}
+
+void w4a16_tile(int tile, int& rows, int& cols) {
+  rows = tile >= 0 ? kTiles[tile].tm : tile == W4A16_WS ? 192 : 256;
+  cols = tile >= 0 ? kTiles[tile].tn : 256;
 }
 
 hipError_t launch_w4a16_direct(const GemmSiblings& gs, int G, int tile, bool out_f32, hipStream_t st) {

@@ -89,6 +89,7 @@ SIGNATURES = {
     "svdq_act_xhat_siblings": (_I, [_P, _L, ctypes.POINTER(ActSibling), _I, _I, _I, _I, _I, _I, _I, _P]),
     "svdq_w4a4_gemm_siblings": (_I, [ctypes.POINTER(W4A4Sibling), _I, _I, _I, _I, _I, _I, _P]),
     "svdq_w4a16_gemm_siblings": (_I, [ctypes.POINTER(W4A16Sibling), _I, _I, _I, _I, _I, _P]),
+    "svdq_w4a16_gemm_tile": (_I, [_I, ctypes.POINTER(_I), _I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "svdq_gate_op": (_I, [_I, _P, _P, _P, _L, _P]),
     "svdq_rms_norm_modulate": (_I, [_P, _L, _P, _P, _I, _I, ctypes.c_float, _P, _L, _P]),
     "svdq_residual_rms_norm_modulate": (_I, [_P, _L, _P, _L, _P, _P, _P, _I, _I, ctypes.c_float, _P, _L, _P, _L,
@@ -155,6 +156,14 @@ def call(name: str, *args) -> None:
 
 def version() -> str:
     return load().svdq_version().decode()
+
+
+def w4a16_tile(m: int, ns, k: int, group: int, rtp: int = 32) -> tuple[int, int, int]:
+    """(launches, tile rows, tile columns) of the W4A16 GEMM of layers of ``ns`` columns over M rows
+    (``svdq_w4a16_gemm_tile``)."""
+    rows, cols = _I(), _I()
+    n = load().svdq_w4a16_gemm_tile(m, (_I * len(ns))(*ns), len(ns), k, group, rtp, ctypes.byref(rows), ctypes.byref(cols))
+    return int(n), rows.value, cols.value
 
 
 def w4a4_tile_cols(m: int, n: int, k: int, group: int, operand: int) -> int:

@@ -273,3 +273,19 @@ def test_act_quant_noalloc_scratch_limit(m, k, g, rtp, fits):
         lib.call("svdq_act_quant_noalloc", None, k, fake, fake, 32, None, 0, None, m, k, g, rtp,
                  lib.SVDQ_ACT_OPERAND_E3M2 | lib.SVDQ_ACT_SX_PAIRS, fake, fake, None, None, k, fake, None)
     assert ("device scratch" in str(ei.value)) == (not fits)
+
+
+def test_w4a16_sibling_launch_rule():
+    """Sibling layers run as one launch wherever one costs no more than a launch per layer: the rule
+    prices launches that exist only (there is none of 256 x 256 tiles for several layers)."""
+    attn, ff = (6144, 6144, 1536, 1536), (16384, 16384)
+    for m in (64, 769, 961, 1024, 1921, 2048, 2689, 4097, 4352):
+        assert lib.w4a16_tile(m, attn, 6144, 64)[0] == 1, m
+    for m in (64, 500, 2381):
+        assert lib.w4a16_tile(m, ff, 6144, 64)[0] == 1, m
+    assert lib.w4a16_tile(64, (1536,), 6144, 64) == (1, 32, 128)
+    assert lib.w4a16_tile(2304, (16384,), 6144, 64) == (1, 192, 256)
+    assert lib.w4a16_tile(16384, (16384,), 6144, 64) == (1, 256, 256)
+    for bad in ((0, (64,), 64, 64), (4, (64, 0), 64, 64), (4, (64,), 96, 64), (4, (64,), 64, 32), (4, (1,) * 5, 64, 64)):
+        assert lib.w4a16_tile(*bad)[0] == 0
+    assert lib.w4a16_tile(4, (64,), 64, 64, 40)[0] == 0
