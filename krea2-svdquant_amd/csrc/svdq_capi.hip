@@ -625,19 +625,6 @@ int svdq_w4a16_gemm_epi(const void* xhat, int64_t ldxh, const void* qw, const vo
   return launched(svdq::launch_w4a16(p, group, out_f32 == 1, stream), "w4a16_gemm");
 }
 
-// The launch that takes all the layers, or false where a launch per layer costs less or does not exist.
-static bool w4a16_grouped(const svdq::GemmSiblings& gs, int group, svdq::W4A16Route& r) {
-  r = svdq::w4a16_route(gs);
-  long own = 0;   // cost of a launch per layer
-  for (int i = 0; i < gs.count; ++i) {
-    svdq::GemmSiblings one{};
-    one.count = 1;
-    one.layer[0] = gs.layer[i];
-    own += svdq::w4a16_route(one).cost;
-  }
-  return fast_group(group) && r.tile != svdq::W4A16_WIDE && r.cost <= own;
-}
-
 int svdq_w4a16_gemm_tile(int M, const int* N, int count, int K, int group, int RTp, int* rows, int* cols) {
   if (!N || count < 1 || count > SVDQ_MAX_SIBLINGS || M <= 0 || K <= 0 || !fast_group(group) || K % group || RTp <= 0 ||
       RTp % 32)
@@ -649,12 +636,14 @@ int svdq_w4a16_gemm_tile(int M, const int* N, int count, int K, int group, int R
     gs.layer[i] = gemm_params(nullptr, nullptr, nullptr, nullptr, RTp, nullptr, M, N[i], K, nullptr, N[i]);
     gs.layer[i].ldxh = K;
   }
-  svdq::W4A16Route r;
-  const int launches = w4a16_grouped(gs, group, r) ? 1 : count;
-  gs.count = 1;
-  if (launches > 1) r = svdq::w4a16_route(gs);
+  int tile = svdq::w4a16_route(gs).tile;
+  const int launches = count == 1 || tile >= svdq::W4A16_WS ? 1 : count;
+  if (launches > 1) {
+    gs.count = 1;
+    tile = svdq::w4a16_route(gs).tile;
+  }
   int tm, tn;
-  svdq::w4a16_tile(r.tile, tm, tn);
+  svdq::w4a16_tile(tile, tm, tn);
   if (rows) *rows = tm;
   if (cols) *cols = tn;
   return launches;
@@ -685,9 +674,10 @@ int svdq_w4a16_gemm_siblings(const svdq_w4a16_sibling* layers, int count, int M,
     tiles += ((M + 191) / 192) * ((l.N + 255) / 256);
   }
   gs.tile0[count] = tiles;
-  if (svdq::W4A16Route r; w4a16_grouped(gs, group, r))
-    return launched(r.tile == svdq::W4A16_WS ? svdq::launch_w4a16_siblings(gs, group, out_f32 == 1, stream)
-                                             : svdq::launch_w4a16_direct(gs, group, r.tile, out_f32 == 1, stream),
+  const int tile = count > 1 && fast_group(group) ? svdq::w4a16_route(gs).tile : svdq::W4A16_WIDE;
+  if (tile >= svdq::W4A16_WS)
+    return launched(tile == svdq::W4A16_WS ? svdq::launch_w4a16_siblings(gs, group, out_f32 == 1, stream)
+                                           : svdq::launch_w4a16_direct(gs, group, tile, out_f32 == 1, stream),
                     "w4a16_gemm_siblings");
   // otherwise one launch per layer, in order, each with its own tile choice
   for (int i = 0; i < count; ++i)

@@ -2370,33 +2370,37 @@ hipError_t launch_w4a16(const GemmParams& p, int G, bool out_f32, hipStream_t st
   const char* ke = getenv("SVDQ_W4A16_KERNEL");
   const long nbn = (p.N + 255) / 256;
   const long tiles_wide = (long)((p.M + 255) / 256) * nbn, tiles192 = (long)((p.M + 191) / 192) * nbn;
-  int route = W4A16_WIDE;
-  if (p.epi || (ke && !strcmp(ke, "wide") && tiles_wide >= 128)) {
-    // Register-staged tiles: with a fused op, and by the environment (tests compare the others with them).
-    if (tiles_wide < 128) {
-      // 128 x 128 (two workgroups of 4 waves per CU) when 256 x 256 tiles leave half the chip idle
-      const dim3 grid(((p.M + 127) / 128) * ((p.N + 127) / 128));
-      if (G == 64) w4a16_kernel<64, 2, false, true><<<grid, 256, 0, st>>>(p);
-      else w4a16_kernel<128, 2, false, true><<<grid, 256, 0, st>>>(p);
-      return hipGetLastError();
+  GemmSiblings one{};
+  one.count = 1;
+  one.layer[0] = p;
+  // Register-staged tiles with a fused op, and by the environment (tests compare the others with them):
+  // 128 x 128 (two workgroups of 4 waves per CU) when 256 x 256 tiles leave half the chip idle.
+  const bool staged = p.epi || (ke && !strcmp(ke, "wide"));
+  const int route = !staged ? w4a16_route(one).tile : tiles_wide < 128 ? W4A16_STAGED : W4A16_WIDE;
+  if (route >= 0) return launch_w4a16_direct(one, G, route, out_f32, st);
+  if (route == W4A16_STAGED) {
+    const dim3 grid(((p.M + 127) / 128) * ((p.N + 127) / 128));
+#define SVDQ_W4A16(GG)                                                                     \
+  if (G == GG) {                                                                          \
+    if (out_f32) w4a16_kernel<GG, 2, true><<<grid, 256, 0, st>>>(p);                       \
+    else if (p.epi) w4a16_kernel<GG, 2, false, true><<<grid, 256, 0, st>>>(p);             \
+    else w4a16_kernel<GG, 2, false><<<grid, 256, 0, st>>>(p);                              \
+    return hipGetLastError();                                                             \
+  }
+    SVDQ_W4A16(64)
+    SVDQ_W4A16(128)
+#undef SVDQ_W4A16
+  }
+  if (route == W4A16_WS) {
+    const dim3 grid((unsigned)tiles192);
+    if (G == 64) {
+      if (out_f32) w4a16_ws_kernel<64, true><<<grid, 512, 0, st>>>(p);
+      else w4a16_ws_kernel<64, false><<<grid, 512, 0, st>>>(p);
+    } else {
+      if (out_f32) w4a16_ws_kernel<128, true><<<grid, 512, 0, st>>>(p);
+      else w4a16_ws_kernel<128, false><<<grid, 512, 0, st>>>(p);
     }
-  } else {
-    GemmSiblings one{};
-    one.count = 1;
-    one.layer[0] = p;
-    route = w4a16_route(one).tile;
-    if (route >= 0) return launch_w4a16_direct(one, G, route, out_f32, st);
-    if (route == W4A16_WS) {
-      const dim3 grid((unsigned)tiles192);
-      if (G == 64) {
-        if (out_f32) w4a16_ws_kernel<64, true><<<grid, 512, 0, st>>>(p);
-        else w4a16_ws_kernel<64, false><<<grid, 512, 0, st>>>(p);
-      } else {
-        if (out_f32) w4a16_ws_kernel<128, true><<<grid, 512, 0, st>>>(p);
-        else w4a16_ws_kernel<128, false><<<grid, 512, 0, st>>>(p);
-      }
-      return hipGetLastError();
-    }
+    return hipGetLastError();
   }
   // tile height 256 or 192: the one with the least work per CU, rounds of tiles x tile rows (a
   // round = one tile on each of the 256 CUs); e.g. M = 2304, N = 16384: 576 tiles of 256 rows

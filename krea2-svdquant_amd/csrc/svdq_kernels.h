@@ -108,13 +108,36 @@ hipError_t launch_weight_scale_pairs(const uint16_t* sw, uint32_t* out, int n, i
 // bytes per row)
 hipError_t launch_weight_operand(const uint8_t* qw, uint8_t* qwe, int N, int K, int mode, hipStream_t st);
 hipError_t launch_w4a16(const GemmParams& p, int G, bool out_f32, hipStream_t st);
-// Which kernel runs W4A16 layers over the same rows (no fused op, group 64 or 128) in one launch, by the
-// cost of its rounds of tiles, and that cost: a tile of svdq_w4a16_direct.hip (>= 0), the specialized
-// waves, or (a single layer) the 256-row register-staged tiles.
-constexpr int W4A16_WS = -1, W4A16_WIDE = -2;
+// Microseconds that a GEMM kernel takes for a round of block tiles, n on each of the 256 CUs (us[n - 1], n up to
+// the `slots` that share a CU): fix + k per 1024 columns of K + r per 32 ranks where every CU has its n-th
+// tile, and fix0, k0, r0 where up to the share `flat` of them has one (the others leave clock and memory to
+// those).
+// The tables are least-squares fits to the kernels' times over tile counts of 1 to 2048, K of 128 to 16384
+// and ranks of 32 to 256.
+struct RoundCost {
+  float fix, k, r, fix0, k0, r0;
+};
+inline float rounds_us(const RoundCost* us, int slots, float flat, long tiles, int K, int RTp) {
+  const float k = K / 1024.0f, r = RTp / 32.0f;
+  const long whole = tiles / (256 * slots), rest = tiles % (256 * slots);
+  const RoundCost& f = us[slots - 1];
+  float t = whole * (f.fix + f.k * k + f.r * r);
+  if (rest) {
+    const long n = (rest - 1) / 256;
+    const float fill = (rest - 256 * n) / 256.0f, q = fill > flat ? (fill - flat) / (1.0f - flat) : 0.0f;
+    const RoundCost& p = us[n];
+    t += q * (p.fix + p.k * k + p.r * r) + (1.0f - q) * (p.fix0 + p.k0 * k + p.r0 * r);
+  }
+  return t;
+}
+// Which kernel runs a W4A16 layer, or sibling layers over the same rows (no fused op, group 64 or 128), and its
+// time in us by its rounds: a tile of svdq_w4a16_direct.hip (>= 0), the specialized waves, or (a single layer)
+// the 256-row or the 128 x 128 register-staged tiles.  For siblings a negative tile other than the specialized
+// waves' means a launch per layer, each by its own rule.
+constexpr int W4A16_WS = -1, W4A16_WIDE = -2, W4A16_STAGED = -3;
 struct W4A16Route {
   int tile;
-  long cost;
+  float us;
 };
 W4A16Route w4a16_route(const GemmSiblings& gs);
 void w4a16_tile(int tile, int& rows, int& cols);   // its block tile

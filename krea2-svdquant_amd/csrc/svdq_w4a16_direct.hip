@@ -5,7 +5,7 @@
 // Same operands, arithmetic and order as the tiles that stage the dequantized weights through LDS
 // (svdq_gemm.hip): 16 columns of K per bf16 MFMA in order, then hi and lo low-rank products 16 ranks at
 // a time, bias, one rounding.  Every output has the same bits on every kernel.
-#include <climits>
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -329,13 +329,44 @@ __global__ void __launch_bounds__(512) w4a16_direct_kernel(GemmSiblings gs) {
 
 struct Tile {
   const char* name;
-  int tm, tn, cost;
+  int tm, tn, slots;
+  RoundCost us[2];   // within 3-5% of the measured times in the root mean square
+  float flat = 0.5f;
 };
-// cost: microseconds of a round, one tile on each of the 256 CUs, at K = 6144 (all kernels scale with K)
-constexpr Tile kTiles[] = {{"32x128", 32, 128, 31}, {"64x128", 64, 128, 35}, {"128x128", 128, 128, 54},
-                           {"192x128", 192, 128, 72}, {"128x256", 128, 256, 92}};
-constexpr int kWsCost = 140, kWideCost = 183;   // 192 x 256 on specialized waves, 256 x 256 register-staged
+constexpr Tile kTiles[] = {
+    {"32x128", 32, 128, 1, {{1.81f, 3.92f, 0.70f, 1.71f, 3.70f, 0.68f}}},
+    {"64x128", 64, 128, 2, {{2.19f, 5.15f, 1.12f, 2.00f, 4.58f, 1.11f}, {1.95f, 9.38f, 2.00f, 2.12f, 8.44f, 2.03f}}},
+    {"128x128", 128, 128, 1, {{3.29f, 8.17f, 1.99f, 3.32f, 6.13f, 1.98f}}},
+    {"192x128", 192, 128, 1, {{3.99f, 11.05f, 3.24f, 4.59f, 7.54f, 2.90f}}},
+    {"128x256", 128, 256, 1, {{5.21f, 14.11f, 2.54f, 5.82f, 9.77f, 2.34f}}},
+};
 constexpr int kTileCount = sizeof(kTiles) / sizeof(kTiles[0]);
+// the older kernels (svdq_gemm.hip): specialized waves, and register-staged
+constexpr Tile kWs = {"192x256", 192, 256, 1, {{6.58f, 22.08f, 1.39f, 7.22f, 15.51f, 0.98f}}};
+constexpr Tile kWide = {"256x256", 256, 256, 1, {{6.81f, 31.46f, 4.67f, 8.87f, 6.00f, 4.97f}}, 0.0f};
+constexpr Tile kStaged = {"128x128staged", 128, 128, 2, {{3.90f, 12.94f, 1.38f, 3.51f, 12.18f, 1.38f}, {4.00f, 21.24f, 2.31f, 5.09f, 18.24f, 2.39f}}};
+constexpr float kLaunchUs = 2.0f;   // a further launch
+
+long tile_count(const GemmSiblings& gs, const Tile& t) {
+  long n = 0;
+  for (int i = 0; i < gs.count; ++i)
+    n += ((long)gs.layer[i].M + t.tm - 1) / t.tm * (((long)gs.layer[i].N + t.tn - 1) / t.tn);
+  return n;
+}
+float tile_us(const GemmSiblings& gs, const Tile& t) {
+  int rtp = 0;
+  for (int i = 0; i < gs.count; ++i) rtp = std::max(rtp, gs.layer[i].RTp);
+  return rounds_us(t.us, t.slots, t.flat, tile_count(gs, t), gs.layer[0].K, rtp);
+}
+// A direct tile: x_hat beyond what the L2s hold is read again for every column of tiles, at about 7 TB/s
+// (M = 12288, N = 1536, K = 6144 on 192x128: 274 us for 1.8 GB, where its rounds alone would take 220).
+float direct_us(const GemmSiblings& gs, const Tile& t) {
+  float mb = 0.0f;
+  for (int i = 0; i < gs.count; ++i)
+    mb += ((long)gs.layer[i].N + t.tn - 1) / t.tn * (2e-6f * gs.layer[i].M * gs.layer[i].K);
+  const float us = tile_us(gs, t);
+  return 2e-6f * gs.layer[0].M * gs.layer[0].K > 32.0f ? std::max(us, mb / 7.0f) : us;
+}
 
 template <int G, int MI, int NJ, int NBUF>
 hipError_t launch_tile(const GemmSiblings& gs, unsigned tiles, bool out_f32, hipStream_t st) {
@@ -357,16 +388,18 @@ hipError_t launch_g(const GemmSiblings& gs, int tile, unsigned tiles, bool out_f
 
 }  // namespace
 
-// The kernel whose rounds of tiles over the 256 CUs cost least.  Measured (K = 6144, group 64, us; the
-// 256-row or specialized-wave tiles, or, below half a chip of those, 128 x 128 tiles through LDS, against
-// these):  M = 64, N = 1536: 80 / 26 (32x128);  M = 77, N = 16384: 84 / 39 (64x128);  M = 256, N = 6144:
-// 82 / 37 (64x128);  M = 512, N = 6144: 87 / 52 (128x128);  M = 768, N = 8192: 130 / 74 (192x128);  M = 1024,
-// N = 6144: 128 / 84, M = 2304, N = 1536: 88 / 57, M = 2304, N = 3072: 131 / 88, M = 4096, N = 6144: 353 / 283
-// (128x256).  The older kernels keep the shapes that fill their rounds: M = 2304, N = 16384: 416
-// (specialized waves) / 438, M = 16384, N = 16384: 2917 (256 x 256) / 2974.
+// The kernel that takes least by its rounds of tiles; the older ones unless a direct tile gains 3% (10% on the
+// 256 x 256 tiles, which re-read the least where there are many row blocks).  Measured,
+// older / direct, us.  Rank 32, K = 6144:  M = 64, N = 1536: 80 / 26 (32x128);  M = 77, N = 16384: 84 / 39 (64x128);
+// M = 256, N = 6144: 82 / 37 (64x128);  M = 512, N = 6144: 87 / 52 (128x128);  M = 768, N = 8192: 130 / 74 (192x128);
+// M = 1024, N = 6144: 128 / 84, M = 4096, N = 6144: 353 / 283 (128x256).  A direct tile gathers its low-rank operands from 32
+// lines per instruction (192x128: 3.2 us per 32 ranks; specialized waves, by DMA: 1.4), and a small K leaves little
+// of what it gains elsewhere, so rank and K decide too (K, rank; 192x256 or 256x256 / direct): M = 1100, N = 16384: 128,
+// 256 39 / 91; M = 3000, N = 6144: 512, 256 52 / 112; M = 1100, N = 16384: 1536, 128 79 / 98; M = 4352, N = 6144: 6144,
+// 256 403 / 459; M = 4352, N = 16384: 6144, 256 849 / 950.
 // These kernels take byte offsets from the tile's first row and column in 32 bits: rows of x_hat below
-// 2^24 bytes, K below 2^25.  SVDQ_W4A16_TILES=<name> in the environment forces a tile, so that tests can run all
-// on one shape.
+// 2^24 bytes, K below 2^25.  SVDQ_W4A16_TILES=<name> in the environment forces a kernel where it can run, so that
+// tests can run all on one shape.
 W4A16Route w4a16_route(const GemmSiblings& gs) {
   const char* e = getenv("SVDQ_W4A16_TILES");
   const char* ke = getenv("SVDQ_W4A16_KERNEL");
@@ -375,26 +408,40 @@ W4A16Route w4a16_route(const GemmSiblings& gs) {
     ws = ws && w4a16_ws_fits(gs.layer[i]);
     direct = direct && gs.layer[i].ldxh < (1L << 23) && gs.layer[i].K < (1 << 25) && !gs.layer[i].epi;
   }
-  auto rounds = [&](int tm, int tn) {
-    long t = 0;
-    for (int i = 0; i < gs.count; ++i) t += ((long)gs.layer[i].M + tm - 1) / tm * (((long)gs.layer[i].N + tn - 1) / tn);
-    return (t + 255) / 256;
-  };
-  // (sibling layers have no launch of 256 x 256 tiles: WIDE then means each layer by its own rule)
-  W4A16Route best{W4A16_WIDE, gs.count > 1 ? LONG_MAX : kWideCost * rounds(256, 256)};
-  if (gs.count > 1 && ke && !strcmp(ke, "wide")) return best;
-  if (ws && kWsCost * rounds(192, 256) <= best.cost) best = {W4A16_WS, kWsCost * rounds(192, 256)};
+  W4A16Route best{W4A16_WIDE, 0.0f};
+  if (gs.count > 1) {
+    if (ke && !strcmp(ke, "wide")) return best;
+    for (int i = 0; i < gs.count; ++i) {
+      GemmSiblings one{};
+      one.count = 1;
+      one.layer[0] = gs.layer[i];
+      best.us += w4a16_route(one).us + (i ? kLaunchUs : 0.0f);
+    }
+    if (const float c = tile_us(gs, kWs); ws && (c < best.us || (e && !strcmp(e, kWs.name)))) best = {W4A16_WS, c};
+  } else {
+    // 256 x 256 tiles where they fill half the chip, 192 rows where those need fewer rounds x rows
+    const long wide = tile_count(gs, kWide), t192 = tile_count(gs, kWs);
+    if (wide < 128) best = {W4A16_STAGED, tile_us(gs, kStaged)};
+    else if (ws && (t192 + 255) / 256 * 192 < (wide + 255) / 256 * 256) best = {W4A16_WS, tile_us(gs, kWs)};
+    else best = {W4A16_WIDE, tile_us(gs, kWide)};
+    if (e && !strcmp(e, kStaged.name)) return {W4A16_STAGED, best.us};
+    if (e && !strcmp(e, kWide.name)) return {W4A16_WIDE, best.us};
+    if (e && ws && !strcmp(e, kWs.name)) return {W4A16_WS, best.us};
+  }
+  if (e && ws && !strcmp(e, kWs.name)) return best;
+  float most = (best.tile == W4A16_WIDE && gs.count == 1 ? 0.90f : 0.97f) * best.us;
   for (int t = 0; t < kTileCount && direct; ++t) {
-    if (e && !strcmp(e, kTiles[t].name)) return {t, 0};
-    const long c = kTiles[t].cost * rounds(kTiles[t].tm, kTiles[t].tn);
-    if (c < best.cost) best = {t, c};
+    const float c = direct_us(gs, kTiles[t]);
+    if (e && !strcmp(e, kTiles[t].name)) return {t, c};
+    if (c < most) best = {t, c}, most = c;
   }
   return best;
 }
 
 void w4a16_tile(int tile, int& rows, int& cols) {
-  rows = tile >= 0 ? kTiles[tile].tm : tile == W4A16_WS ? 192 : 256;
-  cols = tile >= 0 ? kTiles[tile].tn : 256;
+  const Tile& t = tile >= 0 ? kTiles[tile] : tile == W4A16_WS ? kWs : tile == W4A16_STAGED ? kStaged : kWide;
+  rows = t.tm;
+  cols = t.tn;
 }
 
 hipError_t launch_w4a16_direct(const GemmSiblings& gs, int G, int tile, bool out_f32, hipStream_t st) {

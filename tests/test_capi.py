@@ -281,11 +281,22 @@ def test_w4a16_sibling_launch_rule():
     attn, ff = (6144, 6144, 1536, 1536), (16384, 16384)
     for m in (64, 769, 961, 1024, 1921, 2048, 2689, 4097, 4352):
         assert lib.w4a16_tile(m, attn, 6144, 64)[0] == 1, m
-    for m in (64, 500, 2381):
-        assert lib.w4a16_tile(m, ff, 6144, 64)[0] == 1, m
+    assert lib.w4a16_tile(64, ff, 6144, 64)[0] == 1
     assert lib.w4a16_tile(64, (1536,), 6144, 64) == (1, 32, 128)
     assert lib.w4a16_tile(2304, (16384,), 6144, 64) == (1, 192, 256)
     assert lib.w4a16_tile(16384, (16384,), 6144, 64) == (1, 256, 256)
     for bad in ((0, (64,), 64, 64), (4, (64, 0), 64, 64), (4, (64,), 96, 64), (4, (64,), 64, 32), (4, (1,) * 5, 64, 64)):
         assert lib.w4a16_tile(*bad)[0] == 0
     assert lib.w4a16_tile(4, (64,), 64, 64, 40)[0] == 0
+
+
+def test_w4a16_rule_sees_rank_and_k():
+    """Ranks and short K go to the kernels that move the low-rank operands by DMA, or stage them, where
+    the direct tiles' gathers cost more than their rounds save."""
+    t = lib.w4a16_tile
+    assert t(1100, (16384,), 128, 64, 256)[1:] == (192, 256) and t(3000, (6144,), 512, 64, 256)[1:] == (192, 256)
+    assert t(4352, (6144,), 6144, 64, 256)[1:] == (256, 256) and t(4352, (16384,), 6144, 64, 256)[1:] == (192, 256)
+    assert t(1101, (6144, 6144, 1536, 1536), 512, 64, 128) == (1, 192, 256)
+    assert t(77, (16384,), 6144, 128, 64) == (1, 64, 128) and t(512, (6144,), 6144, 64, 128) == (1, 128, 128)
+    assert t(4096, (6144,), 6144, 64) == (1, 128, 256)
+    assert t(12288, (1536,), 6144, 64) == (1, 192, 256)   # x_hat past the L2s, read again per column of tiles

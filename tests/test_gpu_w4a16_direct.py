@@ -71,3 +71,23 @@ def test_siblings_bit_identical_to_single_layers(dev, monkeypatch, m, k, group):
             monkeypatch.setenv("SVDQ_W4A16_TILES", tile)
         for got, want in zip(ops.w4a16_gemm_siblings(xh, qw, sw, mid, l1, bias, group, False), own):
             assert torch.equal(got, want), tile
+
+
+@pytest.mark.parametrize("m,n,k,group,rank,out_f32", [
+    (1, 130, 64, 64, 32, False), (127, 128, 128, 128, 256, True), (129, 257, 320, 64, 160, False),
+    (300, 1000, 512, 64, 256, False), (513, 640, 1088, 64, 32, True)])
+def test_every_kernel_bit_identical_on_small_grids(dev, monkeypatch, m, n, k, group, rank, out_f32):
+    """Fewer than 128 tiles of 256 x 256: the 128 x 128 register-staged tiles and each other kernel, ranks
+    up to eight chunks of 32."""
+    from krea2_svdquant_amd.kernels.hip import ops
+    print(f"w4a16 kernels: M={m} N={n} K={k} G={group} r={rank} f32={out_f32}", flush=True)
+    o = _operands(dev, m, n, k, group, rank, seed=m + n)
+    monkeypatch.delenv("SVDQ_W4A16_KERNEL", raising=False)
+    monkeypatch.setenv("SVDQ_W4A16_TILES", "128x128staged")
+    want = ops.w4a16_gemm(*o, group, out_f32)
+    assert torch.isfinite(want.float()).all()
+    for tile in [None, "192x256", "256x256"] + TILES:
+        monkeypatch.delenv("SVDQ_W4A16_TILES", raising=False)
+        if tile:
+            monkeypatch.setenv("SVDQ_W4A16_TILES", tile)
+        assert torch.equal(ops.w4a16_gemm(*o, group, out_f32), want), tile
