@@ -208,9 +208,16 @@ int svdq_w4a4_gemm(const void* qa, int operand, const void* sxp, const void* qwe
  * these tiles that 32 x 32 to 128 x 64 tiles run them in less time).  All tilings give
  * bit-identical outputs; the environment variable SVDQ_W4A4_TILES=256x128 or 256x256 overrides
  * the choice (the second only where M, N and K are multiples of 256), as do 32x32, 64x64 and
- * 128x64.  No reference counterpart:
+ * 128x64.  The small tiles' choice depends on the rank as well: this is the answer at ranks up to 32
+ * (svdq_w4a4_gemm_tile takes RTp).  No reference counterpart:
  * a host-side query for callers that report which kernel ran (bench.py, tests). */
 int svdq_w4a4_gemm_tile_cols(int M, int N, int K, int group, int operand);
+
+/* Block tile (*rows x *cols, either may be null) of svdq_w4a4_gemm (count 1) or svdq_w4a4_gemm_siblings
+ * (N[i] columns of layer i) with e3m2 operands, group 64 or 128, RTp as in those calls, no fused op;
+ * returns the number of launches: 1, or count where each layer runs by itself (the tile is then the
+ * first layer's), 0 for other arguments.  A host-side query like svdq_w4a4_gemm_tile_cols. */
+int svdq_w4a4_gemm_tile(int M, const int* N, int count, int K, int group, int RTp, int* rows, int* cols);
 
 /* W4A16 GEMM with fused epilogue: the reference pytorch_sim math (quant/svd.py:119-163;
  * dequantization pack.py:26-44 in bf16) and kernels/triton/generic_int4.py:18-133.

@@ -410,8 +410,27 @@ int svdq_w4a4_gemm(const void* qa, int operand, const void* sxp, const void* qwe
 
 int svdq_w4a4_gemm_tile_cols(int M, int N, int K, int group, int operand) {
   if (operand != SVDQ_OPERAND_E3M2 || !fast_group(group) || M <= 0 || N <= 0 || K <= 0 || K % group) return 0;
-  if (svdq::w4a4_small_tile(M, &N, 1, K, group) >= 0) return 0;
+  if (svdq::w4a4_small_tile(M, &N, 1, K, group, 32) >= 0) return 0;
   return group == 64 && svdq::use_wide_tiles(M, N, K) ? 256 : 128;
+}
+
+int svdq_w4a4_gemm_tile(int M, const int* N, int count, int K, int group, int RTp, int* rows, int* cols) {
+  if (!N || count < 1 || count > SVDQ_MAX_SIBLINGS || M <= 0 || K <= 0 || !fast_group(group) || K % group || RTp <= 0 ||
+      RTp % 32)
+    return 0;
+  for (int i = 0; i < count; ++i)
+    if (N[i] <= 0) return 0;
+  int tile = svdq::w4a4_small_tile(M, N, count, K, group, RTp);
+  const int launches = tile >= 0 || K % 512 == 0 ? 1 : count;
+  if (launches > 1) tile = svdq::w4a4_small_tile(M, N, 1, K, group, RTp);
+  int tm = 256, tn = 128;
+  if (tile >= 0) svdq::w4a4_small_tile_size(tile, tm, tn);
+  else if (group == 64 && (count == 1 || launches > 1 ? svdq::use_wide_tiles(M, N[0], K)
+                                                      : svdq::siblings_use_wide_tiles(M, N, count, K)))
+    tn = 256;
+  if (rows) *rows = tm;
+  if (cols) *cols = tn;
+  return launches;
 }
 
 // Checks of one W4A4 layer's arguments and its kernel parameters (no fused op yet).
@@ -479,10 +498,13 @@ int svdq_w4a4_gemm_siblings(const svdq_w4a4_sibling* layers, int count, int oper
     tiles += ((M + 255) / 256) * ((l.N + 127) / 128);
   }
   gs.tile0[count] = tiles;
-  int ns[SVDQ_MAX_SIBLINGS];
-  for (int i = 0; i < count; ++i) ns[i] = layers[i].N;
+  int ns[SVDQ_MAX_SIBLINGS], rtp = 0;
+  for (int i = 0; i < count; ++i) {
+    ns[i] = layers[i].N;
+    rtp = layers[i].RTp > rtp ? layers[i].RTp : rtp;
+  }
   if (operand == SVDQ_OPERAND_E3M2 && fast_group(group) &&
-      (K % 512 == 0 || svdq::w4a4_small_tile(M, ns, count, K, group) >= 0))
+      (K % 512 == 0 || svdq::w4a4_small_tile(M, ns, count, K, group, rtp) >= 0))
     return launched(svdq::launch_w4a4_siblings(gs, group, out_f32 == 1, stream), "w4a4_gemm_siblings");
   // other formats, groups and K: one launch per layer, in order
   for (int i = 0; i < count; ++i)

@@ -2150,6 +2150,18 @@ bool use_wide_tiles(int M, int N, int K) {
   return wide_tiles_pay(bm * (N / 256), bm * (N / 128));
 }
 
+// every layer takes the wide tiles and they pay over the whole launch
+bool siblings_use_wide_tiles(int M, const int* N, int count, int K) {
+  long wide = 0, tiles = 0;
+  for (int i = 0; i < count; ++i) {
+    if (!wide_tiles_apply(M, N[i], K)) return false;
+    wide += (long)(M / 256) * (N[i] / 256);
+    tiles += (long)(M / 256) * ((N[i] + 127) / 128);
+  }
+  const int o = tile_override();
+  return o ? o == 2 : wide_tiles_pay(wide, tiles);
+}
+
 hipError_t launch_w4a4_any_group(const GemmParams& p, int G, bool out_f32, hipStream_t st) {
   if (G <= 0 || G % 16 || p.K % G || p.K % 64) return hipErrorInvalidValue;
   const dim3 grid(((p.M + 127) / 128) * ((p.N + 127) / 128));
@@ -2175,7 +2187,7 @@ hipError_t launch_w4a4(const GemmParams& p, int G, int mode, bool out_f32, hipSt
 #undef SVDQ_W4A4
   if (mode == 2) {
     if (!p.epi) {
-      if (const int small = w4a4_small_tile(p.M, &p.N, 1, p.K, G); small >= 0) {
+      if (const int small = w4a4_small_tile(p.M, &p.N, 1, p.K, G, p.RTp); small >= 0) {
         GemmSiblings one{};
         one.count = 1;
         one.layer[0] = p;
@@ -2229,9 +2241,12 @@ hipError_t launch_w4a4(const GemmParams& p, int G, int mode, bool out_f32, hipSt
 hipError_t launch_w4a4_siblings(const GemmSiblings& gs, int G, bool out_f32, hipStream_t st) {
   if (gs.count < 1 || gs.count > MAX_SIBLINGS) return hipErrorInvalidValue;
   const int K = gs.layer[0].K, M = gs.layer[0].M;
-  int ns[MAX_SIBLINGS];
-  for (int i = 0; i < gs.count; ++i) ns[i] = gs.layer[i].N;
-  if (const int small = w4a4_small_tile(M, ns, gs.count, K, G); small >= 0)
+  int ns[MAX_SIBLINGS], rtp = 0;
+  for (int i = 0; i < gs.count; ++i) {
+    ns[i] = gs.layer[i].N;
+    rtp = std::max(rtp, gs.layer[i].RTp);
+  }
+  if (const int small = w4a4_small_tile(M, ns, gs.count, K, G, rtp); small >= 0)
     return launch_w4a4_small(gs, G, small, out_f32, st);
   int tiles = 0;
   for (int i = 0; i < gs.count; ++i) {
@@ -2249,15 +2264,7 @@ hipError_t launch_w4a4_siblings(const GemmSiblings& gs, int G, bool out_f32, hip
   }
   ch = ch && ch_ok;
   if (G == 64) {
-    // the wide tiles when every layer takes them and they pay over the whole launch
-    bool apply = true;
-    long wide = 0;
-    for (int i = 0; i < gs.count; ++i) {
-      apply = apply && wide_tiles_apply(M, gs.layer[i].N, K);
-      wide += (long)(M / 256) * (gs.layer[i].N / 256);
-    }
-    const int o = tile_override();
-    if (apply && (o ? o == 2 : wide_tiles_pay(wide, tiles))) {
+    if (siblings_use_wide_tiles(M, ns, gs.count, K)) {
       GemmSiblings w = gs;
       int t = 0;
       for (int i = 0; i < gs.count; ++i) {

@@ -354,20 +354,28 @@ __global__ void __launch_bounds__(512) w4a4_e3m2_small_kernel(GemmSiblings gs) {
   w4a4_e3m2_small_tile<G, WM, WN, OUT_F32>(p, t % nbm, t / nbm);
 }
 
-// The tiles, with how many of them share a CU (their LDS) and what 1, 2, 3 of them on every CU take
-// (us at K = 6144, group 64; the ratios hold for group 128 and K = 16384).
+// The tiles, how many of them share a CU (their LDS), and what a round takes with groups of 64 and of 128.
 struct SmallTile {
   const char* name;
   int tm, tn, slots;
-  float us[3];
+  RoundCost us[2][3];
 };
+// (The third 32x32 tile of a CU is priced 15% above its fit: where the rows outgrow the L2s, the operands that
+// such tiles re-read the most come slower than in the fitted grids: M = 2381, N = 256, K = 16384 33 us on 64x64, 49 on 32x32.)
 constexpr SmallTile kSmallTiles[] = {
-    {"32x32", 32, 32, 3, {9.4f, 11.7f, 13.9f}},
-    {"64x64", 64, 64, 1, {13.5f}},
-    {"128x64", 128, 64, 1, {22.5f}},
+    {"32x32", 32, 32, 3,
+     {{{1.85f, 1.09f, 0.38f, 1.50f, 1.00f, 0.35f}, {2.01f, 1.28f, 0.39f, 1.89f, 1.22f, 0.40f}, {1.96f, 2.10f, 0.60f, 2.22f, 1.79f, 0.62f}},
+      {{1.58f, 0.99f, 0.36f, 1.22f, 0.88f, 0.36f}, {1.53f, 1.14f, 0.41f, 1.53f, 1.10f, 0.39f}, {1.77f, 1.92f, 0.55f, 1.93f, 1.59f, 0.58f}}}},
+    {"64x64", 64, 64, 1, {{{2.09f, 1.63f, 0.70f, 1.82f, 1.34f, 0.64f}}, {{1.83f, 1.44f, 0.71f, 1.59f, 1.13f, 0.67f}}}},
+    {"128x64", 128, 64, 1, {{{2.02f, 3.17f, 1.27f, 1.51f, 2.80f, 1.17f}}, {{1.97f, 2.73f, 1.30f, 1.46f, 2.34f, 1.23f}}}},
+};
+constexpr RoundCost kLarge[2] = {{3.70f, 8.59f, 1.08f, 3.10f, 5.95f, 0.64f}, {3.31f, 7.60f, 1.18f, 2.79f, 5.79f, 0.62f}};   // 256 x 128
+constexpr float kLaunchUs = 2.0f;   // a further launch
+struct W4A4Small {
+  int tile;
+  float us;
 };
 constexpr int kSmallCount = sizeof(kSmallTiles) / sizeof(kSmallTiles[0]);
-constexpr int kCUs = 256;
 constexpr int kMaxRows = 1 << 25;
 
 long tile_count(int M, const int* N, int count, int tm, int tn) {
@@ -394,15 +402,31 @@ hipError_t launch_g(const GemmSiblings& gs, int tile, unsigned tiles, bool out_f
   return hipErrorInvalidValue;
 }
 
+// The small tile that takes least, or -1 where the 256 x 128 tiles do; a launch per layer where those do not take
+// siblings (K not a multiple of 512).  Rank 32, K = 6144, small / 256 x 128, us:  M = 64, N = 1536 9.4 / 40.3;
+// M = 128, N = 6144 13.7 / 41.0; M = 256, N = 6144 23.4 / 41.6; M = 512, N = 6144 37.7 / 42.9; M = 1100,
+// N = 1536 24 / 43; and not taken: M = 256, N = 16384 44.8 / 45.3, M = 1024, N = 6144 66 / 50.  Ranks cost a small
+// tile more (128x64: 1.3 us per 32 ranks and round; 256 x 128, through LDS: 1.1 for four times the outputs), and a small K
+// leaves little to gain: M = 512, N = 6144 (64x64 or 128x64 / 256 x 128) at K = 128, rank 256 25 / 12.5; 512, 128
+// 19.6 / 11.7; 1536, 256 31 / 20; 6144, 256 53 / 47; 512, 32 13.1 / 9.4.
+W4A4Small choose(int M, const int* N, int count, int K, int G, int RTp) {
+  const int g = G == 64 ? 0 : 1;
+  W4A4Small best{-1, 0.0f};
+  if (count > 1 && K % 512)
+    for (int i = 0; i < count; ++i) best.us += choose(M, &N[i], 1, K, G, RTp).us + (i ? kLaunchUs : 0.0f);
+  else
+    best.us = rounds_us(&kLarge[g], 1, 0.5f, tile_count(M, N, count, 256, 128), K, RTp);
+  for (int t = 0; t < kSmallCount; ++t) {
+    const SmallTile& k = kSmallTiles[t];
+    const float us = rounds_us(k.us[g], k.slots, 0.5f, tile_count(M, N, count, k.tm, k.tn), K, RTp);
+    if (us < best.us) best = {t, us};
+  }
+  return best;
+}
+
 }  // namespace
 
-// The cheapest small tile by whole rounds over the CUs, or -1 where the 256 x 128 tiles' rounds are
-// within 5% of it: 42 us for a round that leaves CUs idle, up to 52 us for a full one (K = 6144).
-// Measured (small tile / 256 x 128, K = 6144): M = 64, N = 1536 9.4 / 40.3 us; M = 128, N = 6144
-// 13.7 / 41.0; M = 256, N = 6144 23.4 / 41.6; M = 512, N = 6144 37.7 / 42.9; M = 1100, N = 1536 24 /
-// 43; and not taken: M = 256, N = 16384 44.8 / 45.3, M = 1024, N = 6144 66 / 50, M = 2304, N = 1536
-// 45.8 / 44.0.
-int w4a4_small_tile(int M, const int* N, int count, int K, int G) {
+int w4a4_small_tile(int M, const int* N, int count, int K, int G, int RTp) {
   if ((G != 64 && G != 128) || K % G) return -1;
   if (const char* e = getenv("SVDQ_W4A4_TILES")) {   // a tile by name (tests run every tile on one shape)
     for (int t = 0; t < kSmallCount; ++t)
@@ -412,17 +436,12 @@ int w4a4_small_tile(int M, const int* N, int count, int K, int G) {
   // a lane's offset within a stage spans 8 planes of 16 bytes per row, in 32 bits
   for (int i = 0; i < count; ++i)
     if (std::max(M, N[i]) > kMaxRows) return -1;
-  const long large = tile_count(M, N, count, 256, 128);
-  const long whole = large / kCUs, part = large % kCUs;
-  float best = 0.95f * (52.0f * whole + (part ? 42.0f + 10.0f * part / kCUs : 0.0f));
-  int tile = -1;
-  for (int t = 0; t < kSmallCount; ++t) {
-    const SmallTile& k = kSmallTiles[t];
-    const long per_cu = (tile_count(M, N, count, k.tm, k.tn) + kCUs - 1) / kCUs;
-    const float us = (per_cu / k.slots) * k.us[k.slots - 1] + (per_cu % k.slots ? k.us[per_cu % k.slots - 1] : 0.0f);
-    if (us < best) best = us, tile = t;
-  }
-  return tile;
+  return choose(M, N, count, K, G, RTp).tile;
+}
+
+void w4a4_small_tile_size(int tile, int& rows, int& cols) {
+  rows = kSmallTiles[tile].tm;
+  cols = kSmallTiles[tile].tn;
 }
 
 hipError_t launch_w4a4_small(const GemmSiblings& gs, int G, int tile, bool out_f32, hipStream_t st) {

@@ -93,10 +93,13 @@ hipError_t launch_quant_any_group(const uint16_t* xhat, long ldxh, int M, int K,
 hipError_t launch_w4a4(const GemmParams& p, int G, int mode, bool out_f32, hipStream_t st);
 // whether launch_w4a4 (e3m2, group 64, no fused op) runs the 256 x 256 tiles for this shape
 bool use_wide_tiles(int M, int N, int K);
+// the same for a launch of sibling layers
+bool siblings_use_wide_tiles(int M, const int* N, int count, int K);
 // Small block tiles (svdq_gemm_small.hip): which of them runs layers of these widths over M rows in
-// one launch (e3m2, group 64 or 128, no store ops), -1 where the 256-row tiles are the better
-// choice; and the launch (tile0 is recomputed).
-int w4a4_small_tile(int M, const int* N, int count, int K, int G);
+// one launch (e3m2, group 64 or 128, no store ops; RTp the largest of the layers'), -1 where the 256-row
+// tiles are the better choice; and the launch (tile0 is recomputed).
+int w4a4_small_tile(int M, const int* N, int count, int K, int G, int RTp);
+void w4a4_small_tile_size(int tile, int& rows, int& cols);
 hipError_t launch_w4a4_small(const GemmSiblings& gs, int G, int tile, bool out_f32, hipStream_t st);
 // e3m2 operands, G = 64 or 128, K % 512 == 0, every layer without fused store ops
 hipError_t launch_w4a4_siblings(const GemmSiblings& gs, int G, bool out_f32, hipStream_t st);

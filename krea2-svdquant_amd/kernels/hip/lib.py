@@ -89,6 +89,7 @@ SIGNATURES = {
     "svdq_act_xhat_siblings": (_I, [_P, _L, ctypes.POINTER(ActSibling), _I, _I, _I, _I, _I, _I, _I, _P]),
     "svdq_w4a4_gemm_siblings": (_I, [ctypes.POINTER(W4A4Sibling), _I, _I, _I, _I, _I, _I, _P]),
     "svdq_w4a16_gemm_siblings": (_I, [ctypes.POINTER(W4A16Sibling), _I, _I, _I, _I, _I, _P]),
+    "svdq_w4a4_gemm_tile": (_I, [_I, ctypes.POINTER(_I), _I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "svdq_w4a16_gemm_tile": (_I, [_I, ctypes.POINTER(_I), _I, _I, _I, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "svdq_gate_op": (_I, [_I, _P, _P, _P, _L, _P]),
     "svdq_rms_norm_modulate": (_I, [_P, _L, _P, _P, _I, _I, ctypes.c_float, _P, _L, _P]),
@@ -158,12 +159,21 @@ def version() -> str:
     return load().svdq_version().decode()
 
 
-def w4a16_tile(m: int, ns, k: int, group: int, rtp: int = 32) -> tuple[int, int, int]:
-    """(launches, tile rows, tile columns) of the W4A16 GEMM of layers of ``ns`` columns over M rows
-    (``svdq_w4a16_gemm_tile``)."""
+def _tile(fn: str, m: int, ns, k: int, group: int, rtp: int) -> tuple[int, int, int]:
     rows, cols = _I(), _I()
-    n = load().svdq_w4a16_gemm_tile(m, (_I * len(ns))(*ns), len(ns), k, group, rtp, ctypes.byref(rows), ctypes.byref(cols))
+    n = getattr(load(), fn)(m, (_I * len(ns))(*ns), len(ns), k, group, rtp, ctypes.byref(rows), ctypes.byref(cols))
     return int(n), rows.value, cols.value
+
+
+def w4a4_tile(m: int, ns, k: int, group: int, rtp: int = 32) -> tuple[int, int, int]:
+    """(launches, tile rows, tile columns) of the W4A4 e3m2 GEMM of layers of ``ns`` columns over M rows
+    (``svdq_w4a4_gemm_tile``)."""
+    return _tile("svdq_w4a4_gemm_tile", m, ns, k, group, rtp)
+
+
+def w4a16_tile(m: int, ns, k: int, group: int, rtp: int = 32) -> tuple[int, int, int]:
+    """The same for the W4A16 GEMM (``svdq_w4a16_gemm_tile``)."""
+    return _tile("svdq_w4a16_gemm_tile", m, ns, k, group, rtp)
 
 
 def w4a4_tile_cols(m: int, n: int, k: int, group: int, operand: int) -> int:

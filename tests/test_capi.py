@@ -300,3 +300,18 @@ def test_w4a16_rule_sees_rank_and_k():
     assert t(77, (16384,), 6144, 128, 64) == (1, 64, 128) and t(512, (6144,), 6144, 64, 128) == (1, 128, 128)
     assert t(4096, (6144,), 6144, 64) == (1, 128, 256)
     assert t(12288, (1536,), 6144, 64) == (1, 192, 256)   # x_hat past the L2s, read again per column of tiles
+
+
+def test_w4a4_rule_sees_rank_and_k():
+    """The small tiles where their rounds take less, by K and rank; the 256-row tiles elsewhere."""
+    t = lib.w4a4_tile
+    assert t(64, (1536,), 6144, 64) == (1, 32, 32) and t(64, (1536,), 6144, 64, 256) == (1, 32, 32)
+    assert t(256, (6144,), 6144, 64) == (1, 128, 64) and t(256, (6144,), 6144, 64, 128) == (1, 128, 64)
+    assert t(512, (6144,), 6144, 64) == (1, 64, 64) and t(512, (6144,), 6144, 64, 256) == (1, 256, 128)
+    assert t(400, (6144,), 128, 64, 256) == (1, 256, 128) and t(512, (6144,), 512, 128, 64) == (1, 256, 128)
+    assert t(4096, (16384,), 6144, 64) == (1, 256, 256) and t(4352, (6144, 6144, 1536, 1536), 6144, 64) == (1, 256, 256)
+    # siblings at a K that the grouped 256-row tiles do not take: one launch of small tiles, or one per layer
+    assert t(64, (6144, 1536), 320, 64)[0] == 1 and t(4352, (6144, 1536), 320, 64) == (2, 256, 128)
+    for bad in ((0, (64,), 64, 64), (4, (64, 0), 64, 64), (4, (64,), 96, 64), (4, (64,), 64, 32), (4, (1,) * 5, 64, 64)):
+        assert t(*bad)[0] == 0
+    assert t(4, (64,), 64, 64, 40)[0] == 0

@@ -67,3 +67,14 @@ def test_small_tiles_siblings(dev, m, k):
             got = forward_prepared_siblings(x, preps)
         for g, w in zip(got, want):
             assert torch.equal(g, w), tile
+
+
+@pytest.mark.parametrize("m,n,k,group,rank", [(40, 100, 256, 64, 160), (65, 192, 512, 128, 256), (130, 300, 320, 64, 288)])
+def test_small_tiles_large_ranks(dev, m, n, k, group, rank):
+    from krea2_svdquant_amd.kernels.hip.backend import forward_prepared
+    prep, x = _layer(dev, n, k, group, rank, True), _x(dev, m, k)
+    with _tiles("256x128"):
+        want = forward_prepared(x, prep)
+    for tile in ("32x32", "64x64", "128x64", "auto"):
+        with _tiles(tile):
+            assert torch.equal(forward_prepared(x, prep), want), tile
