@@ -111,8 +111,8 @@ __device__ __forceinline__ void smooth64_exact(const u32x4 (&xr)[8], cfloat_ptr 
 // workgroups share a CU; one wave with all 128 columns took 303-433 registers, one workgroup per
 // CU and a second round of workgroups: pass and finalize at M = 2381, K = 16384, rank 64 65.4 -> 37.1
 // us, M = 2381, K = 6144, rank 32 24.2 -> 17.6 us, M = 4096, K = 6144 with 64 + 64 ranks 69 -> 51 us.
-// The build is held to two workgroups per CU (256 registers; four rank tiles then spill, 51 against
-// 56 us without the limit).
+// The build is held to two workgroups per CU (256 registers): three rank tiles then spill 8-15 registers in
+// the e4m3, int8 and packed-code builds, four spill 59 (e3m2; only small inputs take it, see act_quant_run).
 template <int G, int NT, int OPER, bool XHAT, bool QX, bool LX, int NL = 1>
 __device__ __forceinline__ void act_tile(const ActParams* lp) {
   constexpr bool QUANT = OPER != 0, PAIR = G == 128;
@@ -535,7 +535,10 @@ hipError_t launch_act_nt(const ActParams& p, int nt, dim3 grid, hipStream_t st) 
       else act_kernel<G, 2, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p);
       break;
     case 3: act_kernel<G, 3, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p); break;
-    case 4: act_kernel<G, 4, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p); break;
+    case 4:
+      if constexpr (G == 64 || (OPER == 3 && !QX)) act_kernel<G, 4, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p);
+      else return hipErrorInvalidValue;   // (svdq_capi.hip launches fewer)
+      break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

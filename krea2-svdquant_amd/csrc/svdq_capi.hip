@@ -160,13 +160,21 @@ int act_quant_run(const void* x, int64_t ldx, const float* srs, const void* l2, 
   // The first launch quantizes and computes the first 4 column tiles; each further launch adds 4
   // more tiles of the down projections (rank + LoRA rank beyond 128), into their own columns of
   // the split partials.
+  // Quantizing groups of 128, the first launch takes fewer of 4 tiles and more: with 4 it spills (59-129
+  // registers), and a second pass over x costs less.  4 tiles / 2 and then 2, K = 16384, us: M = 512 36 / 30, M = 1024
+  // 46 / 38, M = 2381 92 / 62, M = 4352 168 / 99 (packed codes 224 / 115); 6 tiles as 4 + 2 / 2 + 4 / 3 + 3, M = 4352: 214 / 146 /
+  // 128; 5, 8 and 9 tiles from 2 are as fast or faster than from 3.  Small inputs, e3m2 alone, keep the one launch: M = 64,
+  // K = 6144 15.8 / 17.1, M = 300 17.5 / 18.4, M = 512 19.8 / 19.7.
   p.t0 = 0;
+  int first = nt < 4 ? nt : 4;
+  if (kgroup == 128 && nt >= 4 && !(nt == 4 && e3m2 && !packed && (int64_t)M * K <= 3 << 20))
+    first = nt == 6 || nt == 7 ? 3 : 2;
   if (generic) {   // x_hat and the first tiles, then the group-size-generic quantizer from x_hat
     svdq::ActParams q = p;
     q.qa = nullptr;
     q.sx = nullptr;
     q.qx = nullptr;
-    if (int e = launched(svdq::launch_act(q, 64, nt < 4 ? nt : 4, 0, true, splits, stream),
+    if (int e = launched(svdq::launch_act(q, 64, first, 0, true, splits, stream),
                          "act_quant"))
       return e;
     if (i8) {
@@ -175,12 +183,12 @@ int act_quant_run(const void* x, int64_t ldx, const float* srs, const void* l2, 
                            "act_quant (any-group quantizer)"))
         return e;
     }
-  } else if (int e = launched(svdq::launch_act(p, kgroup, nt < 4 ? nt : 4, e4m3 ? 1 : (i8 ? 2 : (e3m2 ? 3 : 0)),
+  } else if (int e = launched(svdq::launch_act(p, kgroup, first, e4m3 ? 1 : (i8 ? 2 : (e3m2 ? 3 : 0)),
                                                want_xhat, splits, stream),
                               "act_quant")) {
     return e;
   }
-  for (int t0 = 4; t0 < nt; t0 += 4) {
+  for (int t0 = first; t0 < nt; t0 += 4) {
     svdq::ActParams q = p;
     q.t0 = t0;
     q.gps = p.gps * (kgroup / 64);   // the same columns in every split

@@ -361,7 +361,7 @@ struct SmallTile {
   RoundCost us[2][3];
 };
 // (The third 32x32 tile of a CU is priced 15% above its fit: where the rows outgrow the L2s, the operands that
-// such tiles re-read the most come slower than in the fitted grids: M = 2381, N = 256, K = 16384 33 us on 64x64, 49 on 32x32.)
+// such tiles re-read the most come slower than in the fitted grids: M = 2381, N = 256, K = 16384, rank 256 34 us on 64x64, 49 on 32x32.)
 constexpr SmallTile kSmallTiles[] = {
     {"32x32", 32, 32, 3,
      {{{1.85f, 1.09f, 0.38f, 1.50f, 1.00f, 0.35f}, {2.01f, 1.28f, 0.39f, 1.89f, 1.22f, 0.40f}, {1.96f, 2.10f, 0.60f, 2.22f, 1.79f, 0.62f}},

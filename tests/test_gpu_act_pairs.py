@@ -36,3 +36,37 @@ def test_codes_scales_and_down_projection(dev, m, k, rank, extreme):
         bound = np.abs(np.asarray(x_hat, np.float64)) @ np.abs(np.asarray(st.l2, np.float64)).T * (k * 2.0 ** -24 + 2.0 ** -16)
         err = np.abs(ops.mid_values(mid).cpu().numpy()[:, :rank] - want)
         assert np.all(err <= bound + 1e-30)
+
+
+# rank tiles of 32 split over launches: 4 (one launch up to M K = 3 << 20, then 2 + 2), 5 (2 + 3), 6 (3 + 3), 7 (3 + 4) and
+# 9 (2 + 4 + 3), with and without LoRA tiles among the first
+@pytest.mark.parametrize("m,k,r,rl", [(70, 1280, 128, 0), (700, 6144, 128, 0), (700, 6144, 32, 96), (65, 640, 160, 0),
+                                      (129, 1280, 64, 128), (64, 640, 192, 32), (33, 384, 256, 32)])
+@pytest.mark.parametrize("fmt,packed", [("e3m2", False), ("e3m2", True), ("i8", False), ("e4m3", False)])
+def test_rank_tiles_over_launches(dev, m, k, r, rl, fmt, packed):
+    """Codes and scales as with one rank tile; the down projections within the bound of sums of K
+    products in any order."""
+    from krea2_svdquant_amd.kernels.hip import ops
+    print(f"rank tiles: M={m} K={k} r={r}+{rl} {fmt} packed={packed}", flush=True)
+    gen = torch.Generator(device=dev).manual_seed(m + r)
+    x = torch.randn(m, k, device=dev, generator=gen).to(torch.bfloat16)
+    s = (torch.rand(k, device=dev, generator=gen) + 0.5).to(torch.bfloat16)
+    srs = ops.prepare_smooth(s)
+    l2 = (torch.randn(r, k, device=dev, generator=gen) * 0.05).to(torch.bfloat16)
+    down = (torch.randn(rl, k, device=dev, generator=gen) * 0.05).to(torch.bfloat16) if rl else None
+    mult = torch.linspace(0.5, 1.5, rl, device=dev) if rl else None
+    op = ops.OPERAND_NAMES[fmt]
+    one = ops.act_quant(x, srs, l2[:32].contiguous(), None, None, 128, 32, op, packed, False, False, True)
+    got = ops.act_quant(x, srs, l2, down, mult, 128, ops.rank_padded(r + rl), op, packed, False, False, True)
+    qa = [t.cpu().numpy() for t in (one[0], got[0])]
+    if fmt == "e3m2":   # (an odd row count pads the planes with a row that is not written)
+        qa = [e3m2_codes_of(t, m, k) for t in qa]
+    assert np.array_equal(*qa) and all(torch.equal(a, b) for a, b in zip(one[1:3], got[1:3]))
+    xh = (x.float() / s.float()).to(torch.bfloat16).double()
+    want, mag = xh @ l2.double().T, xh.abs() @ l2.double().abs().T
+    if rl:
+        want = torch.cat((want, mult.double() * (x.double() @ down.double().T)), 1)
+        mag = torch.cat((mag, mult.double() * (x.double().abs() @ down.double().abs().T)), 1)
+    v = ops.mid_values(got[4]).double()
+    assert bool(((v[:, : r + rl] - want).abs() <= mag * (k * 2.0 ** -24 + 2.0 ** -16)).all())
+    assert not v[:, r + rl:].any()
