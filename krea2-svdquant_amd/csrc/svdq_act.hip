@@ -530,8 +530,11 @@ hipError_t launch_act_nt(const ActParams& p, int nt, dim3 grid, hipStream_t st) 
   switch (nt) {
     case 1: act_kernel<G, 1, OPER, XHAT, QX, MIDONLY><<<grid, 256, 0, st>>>(p); break;
     case 2:
-      // two rank tiles (ranks 33-64) without LoRA: x prefetched a group ahead as with one tile
-      if (!MIDONLY && p.rl == 0) act_kernel<G, 2, OPER, XHAT, QX, MIDONLY><<<grid, 256, 0, st>>>(p);
+      // Two rank tiles (ranks 33-64) without LoRA: x prefetched a group ahead as with one tile.  Group 64
+      // with e3m2 or int8 codes or x_hat up to 4096 rows, past which the loads evict each other (K = 16384, prefetched
+      // / not, us: e3m2 M = 1024 22.7 / 25.5, M = 4352 55.5 / 52.4, M = 16384 235 / 202; x_hat M = 8192 214 / 185; but
+      // group 128, M = 4352 58.5 / 60.8 and e4m3, M = 12288, K = 6144 to 15360 2 to 5% faster prefetched).
+      if (!MIDONLY && p.rl == 0 && (G == 128 || OPER == 1 || p.M < 4096)) act_kernel<G, 2, OPER, XHAT, QX, MIDONLY><<<grid, 256, 0, st>>>(p);
       else act_kernel<G, 2, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p);
       break;
     case 3: act_kernel<G, 3, OPER, XHAT, QX, true><<<grid, 256, 0, st>>>(p); break;

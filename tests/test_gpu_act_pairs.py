@@ -70,3 +70,21 @@ def test_rank_tiles_over_launches(dev, m, k, r, rl, fmt, packed):
     v = ops.mid_values(got[4]).double()
     assert bool(((v[:, : r + rl] - want).abs() <= mag * (k * 2.0 ** -24 + 2.0 ** -16)).all())
     assert not v[:, r + rl:].any()
+
+
+@pytest.mark.parametrize("m", [4095, 4096, 4100])
+def test_two_rank_tiles_around_the_prefetch_limit(dev, m):
+    """Group 64, ranks 33-64: x is prefetched up to 4096 rows; the same codes, x_hat and sums either way, so
+    the rows that both sides hold have the same bits (K = 256: one split for any M)."""
+    from krea2_svdquant_amd.kernels.hip import ops
+    gen = torch.Generator(device=dev).manual_seed(7)
+    k = 256
+    x = torch.randn(4100, k, device=dev, generator=gen).to(torch.bfloat16)
+    srs = ops.prepare_smooth((torch.rand(k, device=dev, generator=gen) + 0.5).to(torch.bfloat16))
+    l2 = (torch.randn(48, k, device=dev, generator=gen) * 0.05).to(torch.bfloat16)
+    for op, xhat in ((ops.OPERAND_NONE, True), (ops.OPERAND_I8, False)):
+        few = ops.act_quant(x[:64].contiguous(), srs, l2, None, None, 64, 64, op, False, xhat, False)
+        got = ops.act_quant(x[:m].contiguous(), srs, l2, None, None, 64, 64, op, False, xhat, False)
+        for i in (0, 1, 3):
+            assert got[i].numel() == 0 or torch.equal(got[i][:64], few[i])
+        assert torch.equal(ops.mid_values(got[4])[:64], ops.mid_values(few[4]))
