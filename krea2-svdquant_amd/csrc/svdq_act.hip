@@ -414,7 +414,7 @@ __global__ void __launch_bounds__(256) act_shared_x_kernel(ActSiblings s) {
 // [M, 2, RTp] (the bf16 MFMA operands of mid @ l1cat^T).  One thread per 4 columns of a row, eight
 // partials in flight: the launch is a few memory latencies long (M = 64, 24 splits: pass and finalize
 // 11.4 us with 8 columns per thread and four partials in flight, 8.8 us so).
-constexpr int kFinalizeThreads = 128;
+constexpr int kFinalizeThreads = 256;   // at most; half of them while that leaves CUs without a workgroup
 __device__ __forceinline__ void mid_finalize_rows(const float* __restrict__ part, int S, int M, int RTp,
                                                   uint16_t* __restrict__ midp) {
   const int chunks = RTp / 4;
@@ -424,16 +424,22 @@ __device__ __forceinline__ void mid_finalize_rows(const float* __restrict__ part
   const int c = (int)(idx % chunks);
   const long plane = (long)M * RTp;
   const float* src = part + m * RTp + 4 * c;
-  // past the last split the last one again, not added
   f32x4 v = *reinterpret_cast<const f32x4*>(src);
-  for (int s0 = 1; s0 < S; s0 += 8) {
+  int s = 1;
+  for (; s + 8 <= S; s += 8) {
     f32x4 a[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] = *reinterpret_cast<const f32x4*>(src + (long)min(s0 + j, S - 1) * plane);
+    for (int j = 0; j < 8; ++j) a[j] = *reinterpret_cast<const f32x4*>(src + (s + j) * plane);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (s0 + j < S) v += a[j];
+    for (int j = 0; j < 8; ++j) v += a[j];
   }
+  f32x4 a[7];   // the last ones, as many as there are (S is the same for every thread)
+#pragma unroll
+  for (int j = 0; j < 7; ++j)
+    if (s + j < S) a[j] = *reinterpret_cast<const f32x4*>(src + (s + j) * plane);
+#pragma unroll
+  for (int j = 0; j < 7; ++j)
+    if (s + j < S) v += a[j];
   u32x2 hi, lo;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -581,10 +587,13 @@ hipError_t launch_act(const ActParams& p, int G, int nt, int oper, bool xhat, in
   return hipErrorInvalidValue;
 }
 
+static int finalize_threads(long n) { return n > 256L * kFinalizeThreads ? kFinalizeThreads : kFinalizeThreads / 2; }
+
 static hipError_t launch_finalize_siblings(const ActSiblings& s, int splits, hipStream_t st) {
   const long n = (long)s.layer[0].M * (s.layer[0].RTp / 4);
-  const dim3 grid((unsigned)((n + kFinalizeThreads - 1) / kFinalizeThreads), s.count);
-  mid_finalize_siblings_kernel<<<grid, kFinalizeThreads, 0, st>>>(s, splits);
+  const int threads = finalize_threads(n * s.count);
+  const dim3 grid((unsigned)((n + threads - 1) / threads), s.count);
+  mid_finalize_siblings_kernel<<<grid, threads, 0, st>>>(s, splits);
   return hipGetLastError();
 }
 
@@ -640,8 +649,8 @@ hipError_t launch_xhat_siblings(const ActSiblings& s, int nt, int splits, hipStr
 
 hipError_t launch_mid_finalize(const float* part, int S, int M, int RTp, uint16_t* midp, hipStream_t st) {
   const long n = (long)M * (RTp / 4);
-  const unsigned blocks = (unsigned)((n + kFinalizeThreads - 1) / kFinalizeThreads);
-  mid_finalize_kernel<<<blocks, kFinalizeThreads, 0, st>>>(part, S, M, RTp, midp);
+  const int threads = finalize_threads(n);
+  mid_finalize_kernel<<<(unsigned)((n + threads - 1) / threads), threads, 0, st>>>(part, S, M, RTp, midp);
   return hipGetLastError();
 }
 
