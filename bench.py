@@ -304,7 +304,7 @@ def config0_line(args, dev) -> dict:
             "note": "W4A4 forward (activation pass + GEMM with the low-rank epilogue) at M=256 K=N=6144, "
                     "HIP events over 200 back-to-back calls; CPU: the oracle's restatement of the reference "
                     "pytorch_sim forward (bf16 CPU torch, all host threads), median of 5. At this size the "
-                    "GEMM is one row of 48 tiles of 256 x 128 over the 256 CUs"}
+                    "GEMM is two rows of 96 tiles of 128 x 64 over the 256 CUs"}
 
 
 def block_line(args, dev) -> dict:

@@ -10,7 +10,8 @@
 // Layout: a workgroup (4 waves) owns 64 rows and a contiguous range of K-groups (one
 // "split"); wave w takes every 4th group of the range.  Lane l of a wave holds row l, so a
 // group's smoothing scales are the same for the whole wave (scalar loads, SGPR operands) and
-// the group absmax is lane-local.  The 32x32x16 bf16 A operand of the low-rank MFMAs wants
+// the group absmax is lane-local.  (Quantizing groups of 128, a pair of waves takes every 2nd group, 64
+// columns each, and exchanges the rows' maxima through LDS: act_tile.)  The 32x32x16 bf16 A operand of the low-rank MFMAs wants
 // the two 8-column halves of a 16-column slice of one row in lanes l and l+32; one
 // v_permlane32_swap per register turns the lane-per-row data into exactly that for both
 // 32-row tiles.  Per-wave partials are summed in a fixed wave order in LDS and each split
@@ -607,8 +608,8 @@ hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStrea
   // One workgroup per layer, row block and split (blockIdx.z = the layer), or with
   // SVDQ_ACT_SIBLINGS=shared_x x read once for all layers (act_shared_x_kernel; same results, but
   // one wave per SIMD and a quarter of the workgroups: 119 against 79 us for the four attention
-  // inputs at M = 4352, 60 against 44 us for ff.gate / ff.up).  Group 128 with three or four
-  // layers would spill: per layer.
+  // inputs at M = 4352, 60 against 44 us for ff.gate / ff.up).  Group 128 has that build for two layers
+  // only: with three and four it takes 324 and 392 registers, one workgroup per CU.
   const char* e = getenv("SVDQ_ACT_SIBLINGS");
   if (s.count >= 2 && (G == 64 || s.count == 2) && e && !strcmp(e, "shared_x")) {
     const dim3 grid((s.layer[0].M + 63) / 64, splits);
@@ -633,7 +634,7 @@ hipError_t launch_act_siblings(const ActSiblings& s, int G, int splits, hipStrea
 // A pass of each layer by itself starts and ends with CUs idle and brings a finalize of its own, two short
 // launches per layer: bound by latency, so one launch for all takes every set it can (the four attention
 // inputs / ff.up and ff.gate at rank 64 with their GEMMs, group 64, us: 64 rows 72.3 -> 42.5 / 63.5 -> 52.5, 500
-// rows 141 -> 116 / 222.6 -> 213.7, 2381 rows 531 -> 505 / 982 -> 979, 4352 rows 1049 -> 1019 / 1775 -> 1767).
+// rows 141 -> 116 / 222.6 -> 213.7, 2381 rows 531 -> 505 / 982 -> 979).
 hipError_t launch_xhat_siblings(const ActSiblings& s, int nt, int splits, hipStream_t st) {
   if (s.count < 1 || s.count > MAX_SIBLINGS || nt < 1 || nt > 2) return hipErrorInvalidValue;
   for (int i = 0; i < s.count; ++i)   // (act_tile takes a column tile past r as LoRA's)

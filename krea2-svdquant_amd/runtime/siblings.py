@@ -26,10 +26,10 @@ smoothing vector, so the codes differ), then the layers' GEMMs in ONE launch
 M = 4352 the four attention inputs then run 2040 tiles in 8 rounds over the 256 CUs instead of
 3.19 + 0.8 + 0.8 + 3.19 rounds rounded up to 10, and ff.gate + ff.up 4352 tiles in 17 rounds
 instead of 18.  The tiles are the single-layer kernel's, so the outputs are again bit-identical.
-W4A16 layers take the same route (``svdq_w4a16_gemm_siblings``): each layer's x_hat pass, then
-one launch of the specialized-wave kernel's 192 x 256 tiles where its rounds cost no more than
-the layers' own launches: the attention inputs at M = 2304 run 720 tiles in 3 rounds (383 us)
-instead of 538 us in four launches.
+W4A16 layers take the same route (``svdq_w4a16_gemm_siblings``): the x_hat passes in one launch, then
+the GEMMs in one launch of the tile that takes least, where that costs no more than the layers' own
+launches: the attention inputs at M = 4352 run 2040 tiles of 128 x 256, 876 us with their passes
+(978 us as 192 x 256 tiles of the specialized-wave kernel with a pass per layer).
 """
 from __future__ import annotations
 
